@@ -130,7 +130,7 @@ void launch_fold_err(const int* err, int* info, int* sticky, hipStream_t s);
 // Panel (leaf) factorization on the transposed workspace: see panel.hip.
 // xchg (panel_xchg_bytes() bytes) must be zero at the start of a
 // factorization and tagbase must grow by >= 64 from one launch to the next.
-int panel_max_width(int h);  // widest leaf the panel kernel takes at height h
+int panel_max_width(int h, int elem);  // widest leaf the panel kernel takes at height h (elem: bytes of a value)
 size_t panel_xchg_bytes(int max_groups);
 int panel_groups(int h);     // workgroups used at height h (0 = one workgroup, LDS only)
 // mode of a leaf taller than one workgroup holds:

@@ -572,7 +572,7 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
     const int mode = t_safe ? PANEL_TALL : xcd0 ? PANEL_XCD0 : PANEL_PLAIN;
     for (int jj = j; jj < j + jb;) {
       const int h = m - jj;
-      const int w = std::min({leaf, panel_max_width(h), j + jb - jj});
+      const int w = std::min({leaf, panel_max_width(h, (int)sizeof(T)), j + jb - jj});
       mark(pt, fl, LA_PHASE_PANEL, 0);
       c->leaf_tag += 64u;
       int r = K<T>::panel(Tm, ldt, jj, w, m, ipiv, info, c->leaf_tag, xchg, err, mode, st);
@@ -606,7 +606,7 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
     endm(pt, fl);
   };
   // panel 0 on the main stream
-  rc = factor_panel(0, std::min(nb, mn), s, pa, fla, false);
+  rc = factor_panel(0, std::min(nb, mn), s, pa, fla, xcdsplit && panel_groups(m) <= 32);
   if (rc == 0 && n > std::min(nb, mn)) inv_tri(0, std::min(nb, mn), s, pa, fla);
   for (int j = 0; j < mn && rc == 0; j += nb) {
     const int jb = std::min(nb, mn - j);
