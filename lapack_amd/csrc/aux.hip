@@ -50,17 +50,7 @@ void launch_transpose_t(int rows, int cols, const Ti* in, long ld_in, To* out, l
   transpose_kernel<Ti, To, CHECK><<<grid, 256, 0, s>>>(rows, cols, in, ld_in, out, ld_out, ovf, skip);
 }
 
-// ---- row interchanges in the transposed workspace ---------------------------
-// T = A^T: interchanging rows r and p of A is interchanging columns r and p of
-// T.  The panel's interchange sequence ipiv[k1..k2) (SRC/dlaswp.f:156-166 order)
-// is first composed into (dst, src) pairs over the positions it touches --
-// one workgroup walks the sequence once over a position map in LDS -- and the
-// columns are then moved in a single pass: each workgroup owns 16 T rows (one
-// 128-byte line per T column), stages every source value in LDS, barriers,
-// and writes every destination.  Two row ranges (left and right of the panel)
-// are served by one launch.
-constexpr int SWP_ROWS = 16;      // T rows per workgroup
-constexpr int SWP_MAXPAIRS = 512; // 2 * the largest panel width
+constexpr int SWP_MAXPAIRS = 512; // pairs of a composed block of 256 interchanges (at most)
 
 // Composition of one block of K <= 256 interchanges in parallel.  Steps are
 // positions q = b0 .. b0+K-1, step q swapping q with its target p_q >= q
@@ -126,258 +116,6 @@ __device__ void compose_block(int b0, int K, const int* s_p, int* s_r, int* s_ou
     }
   }
   __syncthreads();
-}
-
-// pairs[2q] = dst, pairs[2q+1] = src (0-based positions); *npairs = count.
-// Positions live in [k1, npos).  Up to 256 interchanges that all satisfy
-// p >= q are composed in parallel (compose_block); otherwise one thread walks
-// the sequence over a position map (LDS, or global when it does not fit).
-template <bool LDSMAP>
-__global__ __launch_bounds__(256) void swaps_to_pairs_kernel(int k1, int k2, int npos, const int* __restrict__ ipiv,
-                                                             int* __restrict__ pairs, int* __restrict__ npairs,
-                                                             int* __restrict__ gmap) {
-  extern __shared__ int smem[];
-  __shared__ int s_cnt;
-  __shared__ __align__(16) int s_ip[SWP_MAXPAIRS / 2];
-  __shared__ int s_r[256];
-  __shared__ int s_out[2 * SWP_MAXPAIRS];
-  const int K = k2 - k1;
-  if ((int)threadIdx.x >= K && threadIdx.x < SWP_MAXPAIRS / 2) s_ip[threadIdx.x] = -1;
-  // the sequence itself is read once, in parallel; entries outside [k1, npos)
-  // are ignored, as a self-interchange
-  bool bad = false;
-  for (int x = threadIdx.x; x < K && x < SWP_MAXPAIRS / 2; x += 256) {
-    int p = ipiv[k1 + x] - 1;
-    if (p < k1 || p >= npos) p = k1 + x;
-    if (p < k1 + x) bad = true;
-    s_ip[x] = p;
-  }
-  if (threadIdx.x == 0) s_cnt = 0;
-  if (__syncthreads_or(bad ? 1 : 0) == 0 && K <= 256) {
-    compose_block(k1, K, s_ip, s_r, s_out, &s_cnt);
-    const int np = min(s_cnt, SWP_MAXPAIRS);
-    for (int x = threadIdx.x; x < 2 * np; x += 256) pairs[x] = s_out[x];
-    if (threadIdx.x == 0) *npairs = np;
-    return;
-  }
-  int* cur = LDSMAP ? smem : gmap;
-  const int span = npos - k1;
-  for (int x = threadIdx.x; x < span; x += 256) cur[x] = k1 + x;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = k1; i < k2; ++i) {
-      const int p = i - k1 < SWP_MAXPAIRS / 2 ? s_ip[i - k1] : ipiv[i] - 1;
-      if (p != i && p >= k1 && p < npos) {
-        const int t = cur[i - k1];
-        cur[i - k1] = cur[p - k1];
-        cur[p - k1] = t;
-      }
-    }
-  }
-  __syncthreads();
-  for (int x = threadIdx.x; x < span; x += 256) {
-    const int src = cur[x];
-    if (src != k1 + x) {
-      const int q = atomicAdd(&s_cnt, 1);
-      if (q < SWP_MAXPAIRS) {
-        pairs[2 * q] = k1 + x;
-        pairs[2 * q + 1] = src;
-      }
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) *npairs = min(s_cnt, SWP_MAXPAIRS);
-}
-
-template <class T>
-__global__ __launch_bounds__(256) void apply_pairs_cols_kernel(T* __restrict__ Tm, long ldt, int r0, int r1, int r2,
-                                                               int r3, const int* __restrict__ pairs,
-                                                               const int* __restrict__ npairs, int nblk,
-                                                               int nskip) {
-  // nskip: blocks dispatched to XCDs 0 .. nskip-1 (blockIdx % 8) leave at once
-  int blk = blockIdx.x;
-  if (nskip) {
-    if (blk % 8 < nskip) return;
-    blk = (blk / 8) * (8 - nskip) + (blk % 8 - nskip);
-  }
-  if (blk >= nblk) return;
-  const int np = *npairs;
-  if (np <= 0) return;
-  // this block's 16 rows: first from [r0, r1), then from [r2, r3)
-  const int n1 = (r1 - r0 + SWP_ROWS - 1) / SWP_ROWS;
-  const long c0 = blk < n1 ? (long)r0 + (long)blk * SWP_ROWS : (long)r2 + (long)(blk - n1) * SWP_ROWS;
-  const long cend = blk < n1 ? r1 : r3;
-  const int cl = threadIdx.x & (SWP_ROWS - 1);
-  const int qg = threadIdx.x / SWP_ROWS;  // 16 pair lanes
-  const long c = c0 + cl;
-  const bool ok = c < cend;
-  // every pair of the thread (at most SWP_MAXPAIRS / 16), then every source
-  // in registers, all in flight together; the loads complete and one barrier
-  // (a destination may be another pair's source); then every destination
-  constexpr int QS = 256 / SWP_ROWS, U = SWP_MAXPAIRS / QS;
-  int src[U], dst[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int q = min(qg + QS * u, np - 1);
-    src[u] = pairs[2 * q + 1];
-    dst[u] = pairs[2 * q];
-  }
-  wait_vm();  // all indices here: the source loads below then go out back to back
-  T v[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) v[u] = (ok && qg + QS * u < np) ? Tm[c + (long)src[u] * ldt] : T(0);
-  wait_vm();
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (ok && qg + QS * u < np) Tm[c + (long)dst[u] * ldt] = v[u];
-}
-
-// Everything between two leaves of a panel in one single-workgroup launch
-// (a single workgroup never waits for a share of CUs held by a concurrent
-// trailing update, which a many-workgroup launch does):
-//   1. the leaf's interchanges ipiv[jj..jj+w) (targets in [jj, m), each at
-//      or after its step, as the panel kernels produce them) composed into
-//      pairs (compose_block);
-//   2. the pairs applied to the panel's other T rows, [j, jj) and
-//      [jj+w, jend) (SRC/dgetrf2.f:234-236 on the columns left and right of
-//      the leaf), 64 T rows at a time through registers;
-//   3. the in-panel DTRSM of SRC/dgetrf2.f:240-241 on the columns right of
-//      the leaf: each is solved against the leaf's unit lower triangle by one
-//      thread in the reference's order (BLAS/SRC/dtrsm.f:177-190: for k, skip
-//      a zero x_k, else x_i -= x_k L(i,k) for i > k).
-template <class T>
-__global__ __launch_bounds__(256) void panel_boundary_kernel(T* __restrict__ Tm, long ldt, int j, int jj, int w,
-                                                             int jend, int m, const int* __restrict__ ipiv) {
-  constexpr int W = 64;
-  __shared__ __align__(16) int s_p[256];
-  __shared__ int s_r[256];
-  __shared__ int s_out[2 * SWP_MAXPAIRS];
-  __shared__ int s_cnt;
-  __shared__ T sL[W][W + 1];
-  const int tid = threadIdx.x;
-  s_p[tid] = -1;
-  if (tid < w) {
-    int p = ipiv[jj + tid] - 1;
-    if (p < jj + tid || p >= m) p = jj + tid;  // not of the panel's form: left alone
-    s_p[tid] = p;
-  }
-  if (tid == 0) s_cnt = 0;
-  __syncthreads();
-  compose_block(jj, w, s_p, s_r, s_out, &s_cnt);
-  const int np = min(s_cnt, 2 * W);
-  const int n1 = jj - j, rest = jend - jj - w;
-  const int tot = n1 + rest;
-  // The leaf's triangle (rows [jj, jj+w) are not interchanged here) is read
-  // together with the first chunk of the interchange: L(i,k) = A(jj+i, jj+k)
-  // = T(jj+k, jj+i) -> sL[k][i], zero outside the leaf.
-  T lv[W * W / 256];
-  if (rest > 0) {
-#pragma unroll
-    for (int u = 0; u < W * W / 256; ++u) {
-      const int e = tid + 256 * u;
-      const int k = e % W, i = e / W;
-      lv[u] = (k < w && i < w) ? Tm[(long)(jj + k) + (long)(jj + i) * ldt] : T(0);
-    }
-  }
-  // 64 T rows at a time: every source value of the chunk in registers
-  // (32 per thread), one barrier, every destination (chunks touch disjoint
-  // rows, so the next chunk's loads need no barrier after these stores).
-  // Thread tid moves T row r0 + tid % 64 of pairs tid / 64 + 4u, u < 32:
-  // the same pairs in every chunk, so their indices are read once.
-  constexpr int CH = 64;
-  constexpr int PER = 2 * W * CH / 256;
-  static_assert(256 % CH == 0 && PER * (256 / CH) == 2 * W, "pair lanes");
-  int psrc[PER], pdst[PER];
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int q = tid / CH + (256 / CH) * u;
-    psrc[u] = q < np ? s_out[2 * q + 1] : 0;
-    pdst[u] = q < np ? s_out[2 * q] : 0;
-  }
-  for (int r0 = 0; r0 < tot; r0 += CH) {
-    const int ri = r0 + tid % CH;
-    const bool okr = ri < tot;
-    const long trow = ri < n1 ? (long)j + ri : (long)jj + w + (ri - n1);
-    T v[PER];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int q = tid / CH + (256 / CH) * u;
-      v[u] = (okr && q < np) ? Tm[trow + (long)psrc[u] * ldt] : T(0);
-    }
-    wait_vm();  // every source read before any destination is written
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int q = tid / CH + (256 / CH) * u;
-      if (okr && q < np) Tm[trow + (long)pdst[u] * ldt] = v[u];
-    }
-  }
-  if (rest <= 0) return;
-#pragma unroll
-  for (int u = 0; u < W * W / 256; ++u) {
-    const int e = tid + 256 * u;
-    sL[e % W][e / W] = lv[u];
-  }
-  __syncthreads();
-  if (tid < rest) {
-    const long trow = (long)jj + w + tid;
-    T x[W];
-#pragma unroll
-    for (int i = 0; i < W; ++i) x[i] = i < w ? Tm[trow + (long)(jj + i) * ldt] : T(0);
-    // row k+1 of the triangle is read into registers before row k is
-    // applied, so its LDS reads are in flight while row k's FMAs run (read
-    // inside the branch, only two reads were in flight at a time)
-    T lc[W], ln[W];
-#pragma unroll
-    for (int i = 1; i < W; ++i) lc[i] = sL[0][i];
-#pragma unroll
-    for (int k = 0; k < W; ++k) {
-#pragma unroll
-      for (int i = k + 2; i < W; ++i) ln[i] = sL[k + 1][i];
-      if (x[k] != T(0)) {
-#pragma unroll
-        for (int i = k + 1; i < W; ++i) x[i] = x[i] - x[k] * lc[i];
-      }
-#pragma unroll
-      for (int i = k + 2; i < W; ++i) lc[i] = ln[i];
-    }
-#pragma unroll
-    for (int i = 0; i < W; ++i)
-      if (i < w) Tm[trow + (long)(jj + i) * ldt] = x[i];
-  }
-}
-
-// Row interchanges of a column-major matrix through the same pairs:
-// B(dst, j) <- B_old(src, j); one workgroup per column block of 16.
-template <class T>
-__global__ __launch_bounds__(256) void apply_pairs_rows_kernel(T* __restrict__ B, long ldb, int ncols,
-                                                               const int* __restrict__ pairs,
-                                                               const int* __restrict__ npairs) {
-  const int np = *npairs;
-  if (np <= 0) return;
-  const int j = blockIdx.x * SWP_ROWS + (threadIdx.x & (SWP_ROWS - 1));
-  const int qg = threadIdx.x / SWP_ROWS;
-  const bool ok = j < ncols;
-  // as apply_pairs_cols_kernel: pairs, then sources in registers, one
-  // barrier, every destination
-  constexpr int QS = 256 / SWP_ROWS, U = SWP_MAXPAIRS / QS;
-  int src[U], dst[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int q = min(qg + QS * u, np - 1);
-    src[u] = pairs[2 * q + 1];
-    dst[u] = pairs[2 * q];
-  }
-  wait_vm();
-  T v[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) v[u] = (ok && qg + QS * u < np) ? B[(long)src[u] + (long)j * ldb] : T(0);
-  wait_vm();
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (ok && qg + QS * u < np) B[(long)dst[u] + (long)j * ldb] = v[u];
 }
 
 // ---- DLASWP on a column-major matrix (row interchanges) ----------------------
@@ -806,51 +544,6 @@ int lds_limit() {
   return lds_max;
 }
 
-int swp_max_pairs() { return SWP_MAXPAIRS; }
-
-// (dst, src) pairs of the interchange sequence ipiv[k1..k2) over positions
-// [k1, npos); gmap: npos ints of scratch used when the map does not fit LDS.
-void launch_swaps_to_pairs(int k1, int k2, int npos, const int* ipiv, int* pairs, int* npairs, int* gmap,
-                           hipStream_t s) {
-  const size_t need = sizeof(int) * (size_t)(npos - k1) + 8192;  // + the kernel's static LDS
-  if (need <= (size_t)lds_limit())
-    swaps_to_pairs_kernel<true><<<1, 256, sizeof(int) * (size_t)(npos - k1), s>>>(k1, k2, npos, ipiv, pairs, npairs, gmap);
-  else
-    swaps_to_pairs_kernel<false><<<1, 256, 0, s>>>(k1, k2, npos, ipiv, pairs, npairs, gmap);
-}
-template <class T>
-static void apply_cols_t(T* Tm, long ldt, int r0, int r1, int r2, int r3, const int* pairs, const int* npairs,
-                         hipStream_t s, int nskip) {
-  if (r1 < r0) r1 = r0;
-  if (r3 < r2) r3 = r2;
-  const int nb = (r1 - r0 + SWP_ROWS - 1) / SWP_ROWS + (r3 - r2 + SWP_ROWS - 1) / SWP_ROWS;
-  const int grid = nskip ? (nb + (8 - nskip) - 1) / (8 - nskip) * 8 : nb;
-  if (nb > 0)
-    apply_pairs_cols_kernel<T><<<grid, 256, 0, s>>>(Tm, ldt, r0, r1, r2, r3, pairs, npairs, nb, nskip);
-}
-void launch_apply_pairs_cols_d(double* T, long ldt, int r0, int r1, int r2, int r3, const int* pairs,
-                               const int* npairs, hipStream_t s, int nskip) {
-  apply_cols_t<double>(T, ldt, r0, r1, r2, r3, pairs, npairs, s, nskip);
-}
-void launch_apply_pairs_cols_s(float* T, long ldt, int r0, int r1, int r2, int r3, const int* pairs,
-                               const int* npairs, hipStream_t s, int nskip) {
-  apply_cols_t<float>(T, ldt, r0, r1, r2, r3, pairs, npairs, s, nskip);
-}
-void launch_panel_boundary_d(double* T, long ldt, int j, int jj, int w, int jend, int m, const int* ipiv,
-                             hipStream_t s) {
-  panel_boundary_kernel<double><<<1, 256, 0, s>>>(T, ldt, j, jj, w, jend, m, ipiv);
-}
-void launch_panel_boundary_s(float* T, long ldt, int j, int jj, int w, int jend, int m, const int* ipiv,
-                             hipStream_t s) {
-  panel_boundary_kernel<float><<<1, 256, 0, s>>>(T, ldt, j, jj, w, jend, m, ipiv);
-}
-void launch_apply_pairs_rows_d(double* B, long ldb, int ncols, const int* pairs, const int* npairs, hipStream_t s) {
-  if (ncols > 0) apply_pairs_rows_kernel<double><<<(ncols + SWP_ROWS - 1) / SWP_ROWS, 256, 0, s>>>(B, ldb, ncols, pairs, npairs);
-}
-void launch_apply_pairs_rows_s(float* B, long ldb, int ncols, const int* pairs, const int* npairs, hipStream_t s) {
-  if (ncols > 0) apply_pairs_rows_kernel<float><<<(ncols + SWP_ROWS - 1) / SWP_ROWS, 256, 0, s>>>(B, ldb, ncols, pairs, npairs);
-}
-
 size_t perm_pairs_ints(int k1, int k2) { return k2 > k1 ? (size_t)((k2 - k1 + 255) / 256) * PERM_PB : 0; }
 
 // perm (nrows ints) <- permutation of the interchange sequence; see above.
@@ -934,19 +627,6 @@ void launch_trtri_blocks_s(bool upper, bool unit, int n, int nb, const float* U,
                            long ldw, hipStream_t s) {
   launch_trtri_t<float>(upper, unit, n, nb, U, ldu, W, ldw, s);
 }
-void launch_trtri_uu_d(int nb, const double* U, long ldu, double* W, long ldw, hipStream_t s) {
-  launch_trtri_t<double>(true, true, nb, nb, U, ldu, W, ldw, s);
-}
-void launch_trtri_uu_s(int nb, const float* U, long ldu, float* W, long ldw, hipStream_t s) {
-  launch_trtri_t<float>(true, true, nb, nb, U, ldu, W, ldw, s);
-}
-void launch_trtri_un_d(int nb, const double* U, long ldu, double* W, long ldw, hipStream_t s) {
-  launch_trtri_t<double>(true, false, nb, nb, U, ldu, W, ldw, s);
-}
-void launch_trtri_un_s(int nb, const float* U, long ldu, float* W, long ldw, hipStream_t s) {
-  launch_trtri_t<float>(true, false, nb, nb, U, ldu, W, ldw, s);
-}
-
 static int copy_grid(long work, int nskip) {
   const int g = grid_for(work);
   return nskip ? (g + (8 - nskip) - 1) / (8 - nskip) * 8 : g;

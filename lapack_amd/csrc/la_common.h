@@ -61,26 +61,26 @@ void launch_transpose_s(int rows, int cols, const float* in, long ld_in, float* 
 void launch_transpose_d2s(int rows, int cols, const double* in, long ld_in, float* out, long ld_out,
                           int* overflow, hipStream_t s);
 
-// Row interchanges in the transposed workspace T = A^T (A's rows are T's
-// columns): the sequence ipiv[k1..k2) (1-based entries, applied in order)
-// is composed into at most swp_max_pairs() (dst, src) position pairs over
-// [k1, npos), then applied to T rows [r0, r1) and [r2, r3) in one pass.
-int swp_max_pairs();
-void launch_swaps_to_pairs(int k1, int k2, int npos, const int* ipiv, int* pairs, int* npairs, int* gmap,
-                           hipStream_t s);
-void launch_apply_pairs_cols_d(double* T, long ldt, int r0, int r1, int r2, int r3, const int* pairs,
-                               const int* npairs, hipStream_t s, int nskip = 0);
-void launch_apply_pairs_cols_s(float* T, long ldt, int r0, int r1, int r2, int r3, const int* pairs,
-                               const int* npairs, hipStream_t s, int nskip = 0);
-// Between two leaves of a panel: leaf [jj, jj+w)'s interchanges applied to
-// T rows [j, jj) and [jj+w, jend), then the in-panel DTRSM of T rows
-// [jj+w, jend); one workgroup.  w <= 64.
-void launch_panel_boundary_d(double* T, long ldt, int j, int jj, int w, int jend, int m, const int* ipiv,
-                             hipStream_t s);
-void launch_panel_boundary_s(float* T, long ldt, int j, int jj, int w, int jend, int m, const int* ipiv,
-                             hipStream_t s);
-void launch_apply_pairs_rows_d(double* B, long ldb, int ncols, const int* pairs, const int* npairs, hipStream_t s);
-void launch_apply_pairs_rows_s(float* B, long ldb, int ncols, const int* pairs, const int* npairs, hipStream_t s);
+// Where a leaf's interchanges moved the rows' contents, written by the panel
+// kernels for rows [j0, m) (absolute rows, one int each): leaf[r] the row
+// whose content at the leaf's start is in row r now; pout[r] the same since
+// the panel's start, from the leaf before's pin (null: the panel's first
+// leaf); fin[r] as pout, for the leaf's own rows and, with last, every row.
+struct RowOrg {
+  int* leaf;
+  const int* pin;
+  int* pout;
+  int* fin;
+  int last;
+};
+// A block of w <= 256 factored columns k0 .. on other columns of A (rows of
+// T), see swap_trsm.hip: its interchanges on columns [c0, c1) and [s0, s1),
+// and the solve with its unit lower triangle on [c0, c1).  org: fin of the
+// panel, or leaf of a leaf.
+void launch_swap_trsm_d(double* T, long ldt, int k0, int w, int m, int c0, int c1, int s0, int s1, const int* ipiv,
+                        const int* org, hipStream_t s, int nskip);
+void launch_swap_trsm_s(float* T, long ldt, int k0, int w, int m, int c0, int c1, int s0, int s1, const int* ipiv,
+                        const int* org, hipStream_t s, int nskip);
 // DLASWP on a column-major matrix: perm (nrows ints) <- the permutation of
 // the interchange sequence ipiv[k1..k2-1] (1-based entries, incx = +1/-1),
 // then rows are gathered through it.
@@ -104,13 +104,6 @@ void launch_trtri_blocks_d(bool upper, bool unit, int n, int nb, const double* U
                            long ldw, hipStream_t s);
 void launch_trtri_blocks_s(bool upper, bool unit, int n, int nb, const float* U, long ldu, float* W,
                            long ldw, hipStream_t s);
-// Inverse of the unit upper triangular nb x nb block U (ldu), into W (ldw).
-void launch_trtri_uu_d(int nb, const double* U, long ldu, double* W, long ldw, hipStream_t s);
-void launch_trtri_uu_s(int nb, const float* U, long ldu, float* W, long ldw, hipStream_t s);
-// Inverse of the non-unit upper triangular nb x nb block U, into W.
-void launch_trtri_un_d(int nb, const double* U, long ldu, double* W, long ldw, hipStream_t s);
-void launch_trtri_un_s(int nb, const float* U, long ldu, float* W, long ldw, hipStream_t s);
-
 // Copy a rows x cols column-major block.
 // nskip (copy, interchanges, GEMM, update): no work on XCDs 0 .. nskip-1,
 // which a concurrent panel keeps for itself.
@@ -130,7 +123,6 @@ void launch_fold_err(const int* err, int* info, int* sticky, hipStream_t s);
 // Panel (leaf) factorization on the transposed workspace: see panel.hip.
 // xchg (panel_xchg_bytes() bytes) must be zero at the start of a
 // factorization and tagbase must grow by >= 64 from one launch to the next.
-int panel_max_width(int h, int elem);  // widest leaf the panel kernel takes at height h (elem: bytes of a value)
 size_t panel_xchg_bytes(int max_groups);
 int panel_groups(int h);     // workgroups used at height h (0 = one workgroup, LDS only)
 // mode of a leaf taller than one workgroup holds:
@@ -140,9 +132,9 @@ enum {
   PANEL_TALL = 2,   // column by column over HBM, no workgroup waits for another
 };
 int launch_getf2_panel_d(double* T, long ldt, int j0, int w, int m, int* ipiv, int* info, unsigned tagbase,
-                         double* xchg, int* err, int mode, hipStream_t s);
+                         double* xchg, int* err, int mode, const RowOrg& org, hipStream_t s);
 int launch_getf2_panel_s(float* T, long ldt, int j0, int w, int m, int* ipiv, int* info, unsigned tagbase,
-                         double* xchg, int* err, int mode, hipStream_t s);
+                         double* xchg, int* err, int mode, const RowOrg& org, hipStream_t s);
 
 // Mixed-precision helpers (mp.hip).
 void launch_cast_d2s(int m, int n, const double* A, long lda, float* S, long lds, int* ovf, hipStream_t s);

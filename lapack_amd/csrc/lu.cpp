@@ -14,9 +14,9 @@
 //             (panel.hip), with the in-panel DLASWP / DTRSM / DGEMM between
 //             leaves;
 //   DLASWP    interchanges applied to the columns left and right of the
-//             panel (SRC/dgetrf.f:193,199-200);
-//   DTRSM     U12 = L11^-1 A12 (SRC/dgetrf.f:204-207) as a product with the
-//             inverse of the unit triangle (aux.hip trtri + MFMA GEMM);
+//             panel (SRC/dgetrf.f:193,199-200) and, in the same pass,
+//   DTRSM     U12 = L11^-1 A12 (SRC/dgetrf.f:204-207) on those right of it
+//             (swap_trsm.hip);
 //   DGEMM     A22 -= A21*U12 (SRC/dgetrf.f:212-216) on the FP64 matrix cores.
 // IPIV is the reference's 1-based interchange sequence with absolute rows;
 // INFO the first exact zero pivot.
@@ -319,9 +319,9 @@ template <> struct K<double> {
                         const int* skip = nullptr) {
     launch_transpose_d(r, c, in, li, out, lo, s, skip);
   }
-  static void apply_cols(double* T, long ldt, int r0, int r1, int r2, int r3, const int* pairs, const int* np,
-                         hipStream_t s, int nskip = 0) {
-    launch_apply_pairs_cols_d(T, ldt, r0, r1, r2, r3, pairs, np, s, nskip);
+  static void swap_trsm(double* T, long ldt, int k0, int w, int m, int c0, int c1, int s0, int s1, const int* ipiv,
+                        const int* org, hipStream_t s, int nskip = 0) {
+    launch_swap_trsm_d(T, ldt, k0, w, m, c0, c1, s0, s1, ipiv, org, s, nskip);
   }
   static void gather(int nr, int nc, const int* perm, const double* src, long ls, double* dst, long ld, hipStream_t s,
                      const int* skip = nullptr) {
@@ -339,11 +339,8 @@ template <> struct K<double> {
     launch_copy_d(r, c, src, ls, dst, ld, s, nskip, skip);
   }
   static int panel(double* T, long ldt, int j0, int w, int m, int* ipiv, int* info, unsigned tagbase, double* x,
-                   int* err, int mode, hipStream_t s) {
-    return launch_getf2_panel_d(T, ldt, j0, w, m, ipiv, info, tagbase, x, err, mode, s);
-  }
-  static void boundary(double* T, long ldt, int j, int jj, int w, int jend, int m, const int* ipiv, hipStream_t s) {
-    launch_panel_boundary_d(T, ldt, j, jj, w, jend, m, ipiv, s);
+                   int* err, int mode, const RowOrg& org, hipStream_t s) {
+    return launch_getf2_panel_d(T, ldt, j0, w, m, ipiv, info, tagbase, x, err, mode, org, s);
   }
 };
 // Operand precision of the FP32 factorization's trailing updates on the
@@ -367,9 +364,9 @@ template <> struct K<float> {
                         const int* skip = nullptr) {
     launch_transpose_s(r, c, in, li, out, lo, s, skip);
   }
-  static void apply_cols(float* T, long ldt, int r0, int r1, int r2, int r3, const int* pairs, const int* np,
-                         hipStream_t s, int nskip = 0) {
-    launch_apply_pairs_cols_s(T, ldt, r0, r1, r2, r3, pairs, np, s, nskip);
+  static void swap_trsm(float* T, long ldt, int k0, int w, int m, int c0, int c1, int s0, int s1, const int* ipiv,
+                        const int* org, hipStream_t s, int nskip = 0) {
+    launch_swap_trsm_s(T, ldt, k0, w, m, c0, c1, s0, s1, ipiv, org, s, nskip);
   }
   static void gather(int nr, int nc, const int* perm, const float* src, long ls, float* dst, long ld, hipStream_t s,
                      const int* skip = nullptr) {
@@ -387,11 +384,8 @@ template <> struct K<float> {
     launch_copy_s(r, c, src, ls, dst, ld, s, nskip, skip);
   }
   static int panel(float* T, long ldt, int j0, int w, int m, int* ipiv, int* info, unsigned tagbase, double* x,
-                   int* err, int mode, hipStream_t s) {
-    return launch_getf2_panel_s(T, ldt, j0, w, m, ipiv, info, tagbase, x, err, mode, s);
-  }
-  static void boundary(float* T, long ldt, int j, int jj, int w, int jend, int m, const int* ipiv, hipStream_t s) {
-    launch_panel_boundary_s(T, ldt, j, jj, w, jend, m, ipiv, s);
+                   int* err, int mode, const RowOrg& org, hipStream_t s) {
+    return launch_getf2_panel_s(T, ldt, j0, w, m, ipiv, info, tagbase, x, err, mode, org, s);
   }
 };
 
@@ -466,19 +460,13 @@ static void phase_resolve_locked() {
 }
 
 template <class T>
-size_t getrf_ws_bytes(int m, int n, int nb, int leaf) {
-  (void)leaf;
+size_t getrf_ws_bytes(int m, int n) {
   const long ldt = (long)align_up((size_t)n, 32);
   Carve cv;
   cv.take<T>((size_t)ldt * m);                    // T workspace
-  for (int i = 0; i < 2; ++i) {                   // per stream: TRSM output, triangle inverse, pairs
-    cv.take<T>((size_t)ldt * nb);
-    cv.take<T>((size_t)nb * nb);
-    cv.take<int>((size_t)2 * swp_max_pairs() + 64);
-  }
+  for (int i = 0; i < 5; ++i) cv.take<int>((size_t)m);  // the interchanges' records (RowOrg)
   cv.take<char>(panel_xchg_bytes(0));             // panel exchange + tall-leaf scratch
   cv.take<int>(4);                                // err flag
-  cv.take<int>((size_t)m);                        // position map (fallback)
   return cv.off;
 }
 
@@ -499,9 +487,8 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
   const int nb = tune_nb_for(mn);
   const int leaf = tune_leaf_for(mn);
   const long ldt = (long)align_up((size_t)n, 32);
-  const long ldx = ldt;
   char* ws = nullptr;
-  int rc = ws_acquire(c, getrf_ws_bytes<T>(m, n, nb, leaf), s, &ws);
+  int rc = ws_acquire(c, getrf_ws_bytes<T>(m, n), s, &ws);
   if (rc) return rc;
   if (!c->pstream) {
     // the panel chain (latency-bound) and the trailing update run on two
@@ -519,18 +506,10 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
   LA_TRY(hipStreamWaitEvent(s, c->ev[2], 0));
   Carve cv;
   T* Tm = reinterpret_cast<T*>(ws + cv.take<T>((size_t)ldt * m));
-  T* Xs[2];
-  T* Ws[2];
-  int* Ps[2];
-  for (int i = 0; i < 2; ++i) {
-    Xs[i] = reinterpret_cast<T*>(ws + cv.take<T>((size_t)ldx * nb));
-    Ws[i] = reinterpret_cast<T*>(ws + cv.take<T>((size_t)nb * nb));
-    Ps[i] = reinterpret_cast<int*>(ws + cv.take<int>((size_t)2 * swp_max_pairs() + 64));
-  }
+  int* orgs[5];  // leaf; pin / pout in turn; fin of the panels in turn
+  for (int i = 0; i < 5; ++i) orgs[i] = reinterpret_cast<int*>(ws + cv.take<int>((size_t)m));
   double* xchg = reinterpret_cast<double*>(ws + cv.take<char>(panel_xchg_bytes(0)));
   int* err = reinterpret_cast<int*>(ws + cv.take<int>(4));
-  int* gmap = reinterpret_cast<int*>(ws + cv.take<int>((size_t)m));
-  const long ldw = nb;
   // the multi-workgroup panel owns XCD 0 only on a device of 8 XCDs; a
   // redone call (t_safe) takes the panel form without waits
   const bool xcdsplit = c->xcd8 && env_int("LAPACK_AMD_PANEL_XCD", 1) != 0 && !t_safe;
@@ -564,26 +543,29 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
   K<T>::transpose(m, n, A, lda, Tm, ldt, s);  // T(c, r) = A(r, c)
   endm(pa, fla);
 
+  // the record of panel j's interchanges (read beside the next panel)
+  auto fin_of = [&](int j) { return orgs[3 + ((j / nb) & 1)]; };
   // Panel j: A(j:m, j:j+jb) = T rows j..j+jb, T columns j..m; the DGETRF2
   // recursion flattened to leaves, with in-panel interchanges, DTRSM and
-  // DGEMM between leaves (buffers of slot 1, stream st).
+  // DGEMM between leaves (stream st).
   auto factor_panel = [&](int j, int jb, hipStream_t st, PhaseTimer& pt, std::vector<double>& fl,
                           bool xcd0) -> int {
     const int mode = t_safe ? PANEL_TALL : xcd0 ? PANEL_XCD0 : PANEL_PLAIN;
-    for (int jj = j; jj < j + jb;) {
-      const int h = m - jj;
-      const int w = std::min({leaf, panel_max_width(h, (int)sizeof(T)), j + jb - jj});
+    for (int jj = j, li = 0; jj < j + jb; ++li) {
+      const int w = std::min(leaf, j + jb - jj);
+      const int rest = j + jb - jj - w;
+      const RowOrg org{orgs[0], li == 0 ? nullptr : orgs[1 + ((li + 1) & 1)], orgs[1 + (li & 1)], fin_of(j),
+                       rest == 0 ? 1 : 0};
       mark(pt, fl, LA_PHASE_PANEL, 0);
       c->leaf_tag += 64u;
-      int r = K<T>::panel(Tm, ldt, jj, w, m, ipiv, info, c->leaf_tag, xchg, err, mode, st);
+      int r = K<T>::panel(Tm, ldt, jj, w, m, ipiv, info, c->leaf_tag, xchg, err, mode, org, st);
       endm(pt, fl);
       if (r) return r;
-      const int rest = j + jb - jj - w;
       // interchanges on the panel's other columns and the in-panel DTRSM
-      // (SRC/dgetrf2.f:234-241): one single-workgroup launch
+      // (SRC/dgetrf2.f:234-241)
       if (jj > j || rest > 0) {
         mark(pt, fl, LA_PHASE_LASWP, 0);
-        K<T>::boundary(Tm, ldt, j, jj, w, j + jb, m, ipiv, st);
+        K<T>::swap_trsm(Tm, ldt, jj, w, m, jj + w, j + jb, j, jj, ipiv, orgs[0], st);
         endm(pt, fl);
       }
       // in-panel DGEMM: T(jj+w:j+jb, jj+w:m) -= T(jj+w:j+jb, jj:jj+w) * T(jj:jj+w, jj+w:m)
@@ -598,23 +580,12 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
     return 0;
   };
 
-  // W = inv(L11^T) of panel jp (the DTRSM's triangle) into its buffer;
-  // buffers alternate between consecutive panels
-  auto inv_tri = [&](int jp, int jbp, hipStream_t st, PhaseTimer& pt, std::vector<double>& fl) {
-    mark(pt, fl, LA_PHASE_TRSM, 0);
-    K<T>::trtri_blocks(true, true, jbp, jbp, Tp(jp, jp), ldt, Ws[(jp / nb) & 1], ldw, st);
-    endm(pt, fl);
-  };
   // panel 0 on the main stream
   rc = factor_panel(0, std::min(nb, mn), s, pa, fla, xcdsplit && panel_groups(m) <= 32);
-  if (rc == 0 && n > std::min(nb, mn)) inv_tri(0, std::min(nb, mn), s, pa, fla);
   for (int j = 0; j < mn && rc == 0; j += nb) {
     const int jb = std::min(nb, mn - j);
     if (j > 0) LA_TRY(hipStreamWaitEvent(s, c->ev[0], 0));  // panel j done (panel stream)
-    T* X = Xs[0];
-    T* W = Ws[(j / nb) & 1];
-    int* pairs = Ps[0];
-    int* npairs = pairs + 2 * swp_max_pairs();
+    const int* fin = fin_of(j);
     // Only the next panel's columns are on the critical path: their
     // interchanges, TRSM and update run first and release the panel stream;
     // the interchanges left of the panel and the TRSM / update of the
@@ -623,6 +594,7 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
     const int n2 = n - jn;
     const int jbn = jn < mn ? std::min(nb, mn - jn) : 0;
     const int mrows = m - jn;
+    const int nr = n2 - jbn;
     // the next panel takes XCD 0 for itself (32 workgroups, one per CU) when
     // it runs multi-workgroup; the rest of the step leaves it.  A taller
     // panel (more groups) shares the GPU instead: measured at n = 32768,
@@ -632,45 +604,26 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
     const int npx = (xcdsplit && pg > 0 && pg <= 32) ? 1 : 0;
     const bool split = npx > 0;
     // While the panel holds (nearly) all of XCD 0, every launch beside it
-    // waits for slots there even for the workgroups that only leave: in the
-    // first steps (measured: 28 or more panel workgroups) the rest-of-matrix
-    // DTRSM product then took 5x its time.  There the rest's interchanges,
-    // DTRSM and copy run before the panel, on the whole GPU (those steps are
-    // bound by the trailing update, not by the panel chain).
+    // waits for slots there even for the workgroups that only leave.  There
+    // the rest's interchanges and DTRSM run before the panel, on the whole GPU
+    // (those steps are bound by the trailing update, not by the panel chain).
     const bool pre = split && pg >= pre_pg;
-    // ---- interchanges outside the panel (SRC/dgetrf.f:193,199-200): next panel's columns
-    mark(pa, fla, LA_PHASE_LASWP, 0);
-    if (j > 0 || jn < n) launch_swaps_to_pairs(j, jn, m, ipiv, pairs, npairs, gmap, s);
-    if (jbn > 0) K<T>::apply_cols(Tm, ldt, jn, jn + jbn, 0, 0, pairs, npairs, s);
-    endm(pa, fla);
-    // the triangle's inverse, computed on the panel stream after panel j
-    if (j > 0 && n2 > 0) LA_TRY(hipStreamWaitEvent(s, c->ev[4], 0));
-    if (jbn > 0) {
-      // ---- DTRSM: U12^T = A12^T * inv(L11^T)  (SRC/dgetrf.f:204-207), next panel's columns
-      //      into X (copied back into T after that panel has been released)
-      mark(pa, fla, LA_PHASE_TRSM, 2.0 * jbn * jb * (double)jb / 2.0);
-      K<T>::gemm('N', 'N', jbn, jb, jb, T(1), Tp(jn, j), ldt, W, ldw, T(0), X, ldx, s);
-      endm(pa, fla);
-    }
-    // ---- DGEMM: A22 -= A21*U12, i.e. T22 -= T12 * T21 (SRC/dgetrf.f:212-216),
-    //      the next panel's columns, then that panel on the panel stream
-    const int nr = n2 - jbn;
-    // ---- the rest's interchanges (left of this panel, right of the next one)
-    //      and DTRSM: here, before the next panel, or beside it below
+    // the interchanges left of this panel and right of the next one and the
+    // DTRSM there (SRC/dgetrf.f:193,199-207)
     auto rest_swap_trsm = [&](int nsk) {
-      mark(pa, fla, LA_PHASE_LASWP, 0);
-      if (j > 0 || jn + jbn < n) K<T>::apply_cols(Tm, ldt, 0, j, jn + jbn, n, pairs, npairs, s, nsk);
+      if (j == 0 && nr <= 0) return;
+      mark(pa, fla, LA_PHASE_TRSM, nr > 0 ? (double)nr * jb * jb : 0.0);
+      K<T>::swap_trsm(Tm, ldt, j, jb, m, jn + jbn, n, 0, j, ipiv, fin, s, nsk);
       endm(pa, fla);
-      if (nr > 0) {
-        mark(pa, fla, LA_PHASE_TRSM, 2.0 * nr * jb * (double)jb / 2.0);
-        K<T>::gemm('N', 'N', nr, jb, jb, T(1), Tp(jn + jbn, j), ldt, W, ldw, T(0), X + jbn, ldx, s, nsk);
-        K<T>::copy(nr, jb, X + jbn, ldx, Tp(jn + jbn, j), ldt, s, nsk);
-        endm(pa, fla);
-      }
     };
     if (jbn > 0 && mrows > 0) {
+      mark(pa, fla, LA_PHASE_TRSM, (double)jbn * jb * jb);
+      K<T>::swap_trsm(Tm, ldt, j, jb, m, jn, jn + jbn, 0, 0, ipiv, fin, s);
+      endm(pa, fla);
+      // DGEMM: A22 -= A21*U12, i.e. T22 -= T12 * T21 (SRC/dgetrf.f:212-216),
+      // the next panel's columns, then that panel on the panel stream
       mark(pa, fla, LA_PHASE_GEMM, 2.0 * jbn * (double)mrows * jb);
-      K<T>::update(jbn, mrows, jb, X, ldx, Tp(j, jn), ldt, Tp(jn, jn), ldt, false, s);
+      K<T>::update(jbn, mrows, jb, Tp(jn, j), ldt, Tp(j, jn), ldt, Tp(jn, jn), ldt, 0, s);
       endm(pa, fla);
       if (pre) rest_swap_trsm(0);
       LA_TRY(hipEventRecord(c->ev[1], s));
@@ -678,24 +631,13 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
       rc = factor_panel(jn, jbn, sp, pp, flp, split);
       if (rc) break;
       LA_TRY(hipEventRecord(c->ev[0], sp));
-      // its triangle's inverse, beside the next step's interchanges
-      if (n > jn + jbn) inv_tri(jn, jbn, sp, pp, flp);
-      LA_TRY(hipEventRecord(c->ev[4], sp));
     }
-    if (jbn > 0) {
-      mark(pa, fla, LA_PHASE_TRSM, 0);
-      K<T>::copy(jbn, jb, X, ldx, Tp(jn, j), ldt, s, npx);
-      endm(pa, fla);
-    }
-    // ---- the rest, beside the next panel: interchanges left of this panel
-    //      and right of the next one, their TRSM and update
+    // ---- the rest, beside the next panel
     if (!(pre && jbn > 0 && mrows > 0)) rest_swap_trsm(npx);
-    if (nr > 0) {
-      if (mrows > 0) {
-        mark(pa, fla, LA_PHASE_GEMM, 2.0 * nr * (double)mrows * jb);
-        K<T>::update(nr, mrows, jb, X + jbn, ldx, Tp(j, jn), ldt, Tp(jn + jbn, jn), ldt, npx, s);
-        endm(pa, fla);
-      }
+    if (nr > 0 && mrows > 0) {
+      mark(pa, fla, LA_PHASE_GEMM, 2.0 * nr * (double)mrows * jb);
+      K<T>::update(nr, mrows, jb, Tp(jn + jbn, j), ldt, Tp(j, jn), ldt, Tp(jn + jbn, jn), ldt, npx, s);
+      endm(pa, fla);
     }
   }
   if (rc) {

@@ -4,9 +4,9 @@
 // The panel is A(j0:m-1, j0:j0+w-1) of the matrix being factored, held in the
 // transposed workspace T = A^T, so matrix row r of the panel is T column r and
 // its w values are contiguous.  Three forms, chosen by the panel height h:
-//   * h <= 1024: one workgroup keeps the whole leaf in registers
+//   * h <= 512: one workgroup keeps the whole leaf in registers
 //     (getf2_leaf_kernel);
-//   * 1024 < h <= 32768: G = h/512 workgroups keep it in registers and agree
+//   * 512 < h <= 32768: G = h/512 workgroups keep it in registers and agree
 //     on each column's pivot through a flag-in-data exchange in device memory
 //     (the same kernel; needs its G workgroups resident together);
 //   * taller panels, and every leaf of a factorization being redone after a
@@ -279,6 +279,8 @@ __device__ __forceinline__ u64 ll_word(unsigned payload, unsigned flag) {
 // A touched row has a slot: 0..7 for the group's own rows, 8 + i for the row
 // first touched as step i's pivot; each thread follows its row's slot and the
 // slot its content came from, and a candidate carries the latter.
+// It also follows the row that content was in at the leaf's start (corg),
+// which tells the other columns' interchanges their sources (swap_trsm.hip).
 // What bounds it: the chain A..D (1500-2100 cycles a column in one workgroup,
 // 4200 with 32, 945 of them the exchange's round trip), then E (4000-7000 a
 // group).  With several workgroups only the next group's columns are updated
@@ -291,24 +293,27 @@ template <class T, int W, int NTH, bool MULTI, bool XCD0>
 __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, long ldt, int j0, int w, int m,
                                                         int* __restrict__ ipiv, int* __restrict__ info,
                                                         unsigned tagbase, u64* __restrict__ xbuf,
-                                                        int* __restrict__ err, int Gp, unsigned* __restrict__ ctr) {
+                                                        int* __restrict__ err, int Gp, unsigned* __restrict__ ctr,
+                                                        RowOrg org) {
   constexpr int NW = NTH / 64;
   constexpr int VW = (int)sizeof(T) / 4;      // words of a value
-  constexpr int MW = (LG + 1) * VW + 1;       // words of a candidate
+  constexpr int MW = (LG + 1) * VW + 2;       // words of a candidate
+  constexpr int KW = LG * VW + 2;             // words of row k
   constexpr int NS = MULTI ? GMAX : NW;       // candidates a column folds (at most)
   constexpr int SR = W - LG + 2;              // row stride of s_sw / s_u
   // one workgroup's fold: LPS lanes a candidate, VPL values a lane, the
   // column searched in the candidate's last lane
-  constexpr int LPS = NW >= 16 ? 4 : NW >= 8 ? 8 : 16, VPL = LPS >= LG ? 1 : LG / LPS, LV = LG / VPL;
+  constexpr int LPS = NW >= 8 ? 8 : 16, VPL = LPS >= LG ? 1 : LG / LPS, LV = LG / VPL;
   static_assert(NW * LPS <= 64, "one lane set per wave");
   struct Msg {
     T v[LG];
     T rp;      // 1 / v[step]
     int meta;  // row | content's slot << 16 (NOSLOT: none), or -1: no candidate
+    int org;   // the leaf's row its content was in at the start
   };
   struct RowK {
     T v[LG];
-    int osl;
+    int osl, org;
   };
   __shared__ __align__(16) Msg s_wmsg[2][NW];  // the waves' candidates
   __shared__ __align__(16) Msg s_msg[MULTI ? 2 : 1][MULTI ? NS : 1];
@@ -364,7 +369,7 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
   // The wave's 64 rows in and out through LDS, CP columns at a time: an access
   // of the matrix touches whole runs of CP values of 64 / CP rows (a row a lane
   // would touch 64 lines an instruction).
-  constexpr int CP = NTH >= 1024 ? 8 : 16;
+  constexpr int CP = 16;
   constexpr int RP = 64 / CP;  // rows of one access
   __shared__ T s_stage[NW][64][CP + 1];
   T v[W];
@@ -393,6 +398,7 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
   bool failed = false;
 
   int my_piv = 0;     // lane k: step k's pivot row
+  int corg = lr;      // the leaf's row this row's content was in at the start
   int zero_at = -1;   // the first step with a zero pivot
   const bool valid = lr < h;
   // An exchange word to the other workgroups.  All of them on one XCD share
@@ -463,6 +469,7 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
 #pragma unroll
             for (int c = 0; c < LG; ++c) s_rowk[par].v[c] = v[c];
             s_rowk[par].osl = osl;
+            s_rowk[par].org = corg;
           }
           const unsigned wm = wave_max_recip(hi, v[kk], &rp);
           const int wl = pick_lane<T, 1, 64>(v[kk], cand, lr == k, hi, wm, &none);
@@ -472,6 +479,7 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
             for (int c = 0; c < LG; ++c) ms.v[c] = v[c];
             ms.rp = rp;
             ms.meta = none ? -1 : lr | (osl << 16);
+            ms.org = corg;
           }
         }
         // the wave's own candidate as words, should it be the workgroup's
@@ -482,7 +490,7 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
         }
         __syncthreads();
         // ---- B, C
-        int meta;
+        int meta, porg;
         T uc[LG], rp;  // the pivot row's group values and its pivot's reciprocal (uniform)
         if (MULTI) {
           {
@@ -493,7 +501,7 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
             u64* buf = xbuf + (size_t)par * MSG_PAR;
             if (wave == bw && lane < MW) put(buf + (size_t)b * MSGS + lane, ll_word(mine, flag));
             // row k, which only the owner of the pivot row needs, after the candidate
-            if (top_wave && lane < LG * VW + 1) {
+            if (top_wave && lane < KW) {
               const unsigned x = reinterpret_cast<const unsigned*>(&s_rowk[par])[lane];
               put(buf + (size_t)GMAX * MSGS + lane, ll_word(x, flag));
             }
@@ -516,7 +524,7 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
 #pragma unroll
             for (int q = 0; q < NP; ++q) {
               const int sl = q * SP + (tid >> 5);
-              need[q] = !failed && (sl < G ? wd < MW : (sl == G && wd < LG * VW + 1));
+              need[q] = !failed && (sl < G ? wd < MW : (sl == G && wd < KW));
               x[q] = 0;
             }
             unsigned spins = 0;
@@ -554,12 +562,13 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
           failed = s_fail != 0;
           const bool in = lane < G;
           const Msg& ms = s_msg[par][in ? lane : 0];
-          const int cm = ms.meta;
+          const int cm = ms.meta, co = ms.org;
           const T crp = ms.rp;
           bool none;
           const int ws = pick_lane<T, 1, 64>(ms.v[kk], in && cm >= 0, (cm & 0xffff) == k, &none);
           const T x = s_msg[par][ws].v[lane & (LG - 1)];
           meta = __builtin_amdgcn_readlane(cm, ws);
+          porg = __builtin_amdgcn_readlane(co, ws);
           rp = lane_value(crp, ws);
 #pragma unroll
           for (int c = 0; c < LG; ++c) uc[c] = lane_value(x, c);
@@ -572,11 +581,12 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
           T x[VPL];
 #pragma unroll
           for (int z = 0; z < VPL; ++z) x[z] = ms.v[z * LV + ((lane + (z == H ? kk + 1 : 0)) & (LV - 1))];
-          const int cm = ms.meta;
+          const int cm = ms.meta, co = ms.org;
           const T crp = ms.rp;
           bool none;
           const int wl = pick_lane<T, LPS, NW * LPS>(x[H], cm >= 0, (cm & 0xffff) == k, &none);
           meta = __builtin_amdgcn_readlane(cm, wl);
+          porg = __builtin_amdgcn_readlane(co, wl);
           rp = lane_value(crp, wl);
           const int w0 = wl & ~(LPS - 1);
 #pragma unroll
@@ -600,12 +610,14 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
 #pragma unroll
             for (int c = 0; c < LG; ++c) v[c] = uc[c];
             osl = ts[kk];
+            corg = porg;
           }
           if (p >= wrow0 && p < wrow0 + 64) {
             if (lr == p) {
 #pragma unroll
               for (int c = 0; c < LG; ++c) v[c] = s_rowk[par].v[c];
               osl = s_rowk[par].osl;
+              corg = s_rowk[par].org;
               if (myslot == NOSLOT) myslot = LG + kk;
             }
           }
@@ -780,6 +792,13 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
       for (int c = 0; c < LG; ++c) v[W - LG + c] = t[c];
     }
   }
+  if (lr < h) {
+    const int o = j0 + (corg >= 0 && corg < h ? corg : lr);  // (out of range only after a wait gave up)
+    const int po = org.pin ? org.pin[o] : o;
+    org.leaf[j0 + lr] = o;
+    org.pout[j0 + lr] = po;
+    if (org.last || lr < kmax) org.fin[j0 + lr] = po;
+  }
   if (b == 0 && wave == NW - 1) {
     if (lane < kmax) ipiv[j0 + lane] = j0 + my_piv + 1;
     if (lane == 0 && zero_at >= 0) atomicCAS(info, 0, j0 + zero_at + 1);
@@ -937,13 +956,36 @@ __global__ __launch_bounds__(256) void tall_update_kernel(T* __restrict__ Tm, lo
   if (next_keys) tall_block_max(best, brow, tb);
 }
 
+// The record of the tall form's interchanges (RowOrg), from IPIV: one
+// workgroup, thread 0 walking the at most 64 interchanges.
+__global__ __launch_bounds__(256) void tall_org_kernel(int j0, int kmax, int m, const int* __restrict__ ipiv,
+                                                       RowOrg org) {
+  for (int r = j0 + (int)threadIdx.x; r < m; r += 256) org.leaf[r] = r;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = j0; k < j0 + kmax; ++k) {
+      const int p = ipiv[k] - 1;
+      if (p > k && p < m) {
+        const int t = org.leaf[k];
+        org.leaf[k] = org.leaf[p];
+        org.leaf[p] = t;
+      }
+    }
+  }
+  __syncthreads();
+  for (int r = j0 + (int)threadIdx.x; r < m; r += 256) {
+    const int o = org.leaf[r];
+    const int po = org.pin ? org.pin[o] : o;
+    org.pout[r] = po;
+    if (org.last || r < j0 + kmax) org.fin[r] = po;
+  }
+}
+
 }  // namespace
 
-// Launch configurations: one workgroup with a thread a row up to 1024 rows
-// (fewer threads for the shorter leaves: fewer waves to fold and to wait for);
-// 1024 threads have 128 registers each, which hold 32 FP64 or 64 FP32 columns.
+// Launch configurations: one workgroup with a thread a row up to 512 rows
+// (fewer threads for the shorter leaves: fewer waves to fold and to wait for).
 // Beyond that G workgroups of 512 threads; past GMAX workgroups the tall form.
-int panel_max_width(int h, int elem) { return h > 512 && h <= 1024 && elem == 8 ? 32 : 64; }
 static size_t tall_offset() { return (sizeof(u64) * LL_WORDS + 255) / 256 * 256; }
 // the XCD-0 panel's rank and arrival counters (zeroed with the exchange
 // buffer at the start of a factorization; each launch resets its own)
@@ -951,24 +993,24 @@ static size_t rank_offset() { return tall_offset() + (sizeof(TallBuf) + 255) / 2
 size_t panel_xchg_bytes(int) { return rank_offset() + 256; }
 
 // Workgroups the panel kernel uses at height h (0 = a single workgroup).
-int panel_groups(int h) { return h <= 1024 ? 0 : (h + 511) / 512; }
+int panel_groups(int h) { return h <= 512 ? 0 : (h + 511) / 512; }
 
 // mode: PANEL_PLAIN (G workgroups), PANEL_XCD0 (8*G blocks, those of the
 // first XCDs take part), PANEL_TALL (the form without waits).
 template <class T>
 static int launch_panel_t(T* Tm, long ldt, int j0, int w, int m, int* ipiv, int* info, unsigned tagbase,
-                          double* xchg, int* err, int mode, hipStream_t s) {
+                          double* xchg, int* err, int mode, const RowOrg& org, hipStream_t s) {
   const int h = m - j0;
   if (h <= 0 || w <= 0) return 0;
-  if (w > panel_max_width(h, (int)sizeof(T))) return LA_ERR_LIMIT;
+  if (w > WMAX) return LA_ERR_LIMIT;
   u64* xb = reinterpret_cast<u64*>(xchg);
 #define LA_LEAF(W, NTH, MULTI, XCD0, blocks, g, ctr) \
-  getf2_leaf_kernel<T, W, NTH, MULTI, XCD0><<<blocks, NTH, 0, s>>>(Tm, ldt, j0, w, m, ipiv, info, tagbase, xb, err, g, ctr)
-  if (h <= 1024) {
+  getf2_leaf_kernel<T, W, NTH, MULTI, XCD0><<<blocks, NTH, 0, s>>>(Tm, ldt, j0, w, m, ipiv, info, tagbase, xb, err, g, ctr, \
+                                                              org)
+  if (h <= 512) {
     if (h <= 128) LA_LEAF(64, 128, false, false, 1, 1, nullptr);
     else if (h <= 256) LA_LEAF(64, 256, false, false, 1, 1, nullptr);
-    else if (h <= 512) LA_LEAF(64, 512, false, false, 1, 1, nullptr);
-    else LA_LEAF((sizeof(T) == 8 ? 32 : 64), 1024, false, false, 1, 1, nullptr);
+    else LA_LEAF(64, 512, false, false, 1, 1, nullptr);
     return 0;
   }
   const int G = (h + 511) / 512;
@@ -987,6 +1029,7 @@ static int launch_panel_t(T* Tm, long ldt, int j0, int w, int m, int* ipiv, int*
       tall_update_kernel<T><<<parts(k + 1 < kmax ? k + 1 : k), 256, 0, s>>>(Tm, ldt, j0, k, w, h, tb,
                                                                             k + 1 < kmax ? 1 : 0);
     }
+    tall_org_kernel<<<1, 256, 0, s>>>(j0, kmax, m, ipiv, org);
     return 0;
   }
   if (mode == PANEL_XCD0)
@@ -999,12 +1042,12 @@ static int launch_panel_t(T* Tm, long ldt, int j0, int w, int m, int* ipiv, int*
 }
 
 int launch_getf2_panel_d(double* T, long ldt, int j0, int w, int m, int* ipiv, int* info, unsigned tagbase,
-                         double* xchg, int* err, int mode, hipStream_t s) {
-  return launch_panel_t<double>(T, ldt, j0, w, m, ipiv, info, tagbase, xchg, err, mode, s);
+                         double* xchg, int* err, int mode, const RowOrg& org, hipStream_t s) {
+  return launch_panel_t<double>(T, ldt, j0, w, m, ipiv, info, tagbase, xchg, err, mode, org, s);
 }
 int launch_getf2_panel_s(float* T, long ldt, int j0, int w, int m, int* ipiv, int* info, unsigned tagbase,
-                         double* xchg, int* err, int mode, hipStream_t s) {
-  return launch_panel_t<float>(T, ldt, j0, w, m, ipiv, info, tagbase, xchg, err, mode, s);
+                         double* xchg, int* err, int mode, const RowOrg& org, hipStream_t s) {
+  return launch_panel_t<float>(T, ldt, j0, w, m, ipiv, info, tagbase, xchg, err, mode, org, s);
 }
 
 }  // namespace la
