@@ -600,9 +600,12 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
     // panel (more groups) shares the GPU instead: measured at n = 32768,
     // reserving a second XCD slows the then dominant update more than it
     // speeds the panel (in FP32 as well: DSGESV 467 instead of 406 ms).
+    // The two workgroups of a panel of up to 1024 rows run on XCD 0 as well,
+    // but beside the update: reserving it for them takes an eighth of the GPU
+    // from the update for two CUs.
     const int pg = jbn > 0 ? panel_groups(m - jn) : 0;
-    const int npx = (xcdsplit && pg > 0 && pg <= 32) ? 1 : 0;
-    const bool split = npx > 0;
+    const bool split = xcdsplit && pg > 0 && pg <= 32;
+    const int npx = split && pg > 2 ? 1 : 0;
     // While the panel holds (nearly) all of XCD 0, every launch beside it
     // waits for slots there even for the workgroups that only leave.  There
     // the rest's interchanges and DTRSM run before the panel, on the whole GPU

@@ -430,15 +430,21 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
 #pragma unroll
     for (int i = 0; i < LG; ++i) u[i] = s_u[i][LG * cu + (lane & (LG - 1))];
   };
+  // In FP32 the eight products are summed on their own and added once: one
+  // rounding at the element's size a group instead of eight.
   auto apply_u = [&](const T (&u)[LG], const T (&nl)[LG], T* vq, int r0) {
-    if (top_wave) {
+    constexpr bool SUM = sizeof(T) == 4;
+    if (SUM || top_wave) {
       T t[LG];
 #pragma unroll
-      for (int c = 0; c < LG; ++c) t[c] = vq[c];
+      for (int c = 0; c < LG; ++c) t[c] = SUM ? T(0) : vq[c];
 #pragma unroll
       for (int i = 0; i < LG; ++i) fmac_lanes(t, u[i], nl[i]);
 #pragma unroll
-      for (int c = 0; c < LG; ++c) vq[c] = lr >= r0 ? t[c] : vq[c];
+      for (int c = 0; c < LG; ++c) {
+        const T x = SUM ? vq[c] + t[c] : t[c];
+        vq[c] = !top_wave || lr >= r0 ? x : vq[c];
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < LG; ++i) fmac_lanes(vq, u[i], nl[i]);

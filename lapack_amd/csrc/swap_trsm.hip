@@ -65,17 +65,22 @@ constexpr int SC = 16;        // columns of A a workgroup owns
 constexpr int SWMAX = 256;    // widest block
 constexpr int SNT = 512;
 
-// Steps K .. SB-1 of the substitution: sl[k][i] = -L(i, k).
+// Steps K .. SB-1 of the substitution: sl[k][i] = -L(i, k).  The products of
+// sixteen steps are summed on their own (t) before they join the rows below.
 template <class T, int K>
-__device__ __forceinline__ void solve_steps(T (&x)[SB / 16], const T (*sl)[SB + 1], int sub) {
+__device__ __forceinline__ void solve_steps(T (&x)[SB / 16], T (&t)[SB / 16], const T (*sl)[SB + 1], int sub) {
   if constexpr (K < SB) {
     constexpr int KM = K / 16, KS = K % 16;
-    T t = x[KM];
-    fmac_from<KS>(t, x[KM], sl[K][16 * KM + sub]);
+    T y = x[KM];
+    fmac_from<KS>(y, x[KM], sl[K][16 * KM + sub]);
 #pragma unroll
-    for (int m = KM + 1; m < SB / 16; ++m) fmac_from<KS>(x[m], x[KM], sl[K][16 * m + sub]);
-    x[KM] = sub > KS ? t : x[KM];
-    solve_steps<T, K + 1>(x, sl, sub);
+    for (int m = KM + 1; m < SB / 16; ++m) {
+      if (KS == 0) t[m] = T(0);
+      fmac_from<KS>(t[m], x[KM], sl[K][16 * m + sub]);
+      if (KS == 15) x[m] = x[m] + t[m];
+    }
+    x[KM] = sub > KS ? y : x[KM];
+    solve_steps<T, K + 1>(x, t, sl, sub);
   }
 }
 
@@ -196,7 +201,8 @@ __global__ __launch_bounds__(SNT) void swap_trsm_kernel(T* __restrict__ Tm, long
 #pragma unroll
       for (int z = 0; z < SB / 16; ++z) x[z] = sB[SB * b + 16 * z + sub][cc];
       if (s_odd == 0) {
-        solve_steps<T, 0>(x, sL, sub);
+        T t[SB / 16];
+        solve_steps<T, 0>(x, t, sL, sub);
       } else {
         for (int k = 0; k < SB; ++k) {
           T xk = T(0);
@@ -217,13 +223,11 @@ __global__ __launch_bounds__(SNT) void swap_trsm_kernel(T* __restrict__ Tm, long
       const int t = wave + NW * z;
       if (t < nt) {
         const int i0 = SB * (b + 1) + 16 * t;
-        acc_t acc;
+        acc_t acc = acc_t{};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[r] = sB[i0 + MM::row(lk, r)][li];
+        for (int s = 0; s < 16; ++s) acc = MM::op(a[z][s], sB[SB * b + 16 * lk + s][li], acc);
 #pragma unroll
-        for (int s = 0; s < 16; ++s) acc = MM::op(-a[z][s], sB[SB * b + 16 * lk + s][li], acc);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sB[i0 + MM::row(lk, r)][li] = acc[r];
+        for (int r = 0; r < 4; ++r) sB[i0 + MM::row(lk, r)][li] -= acc[r];
       }
     }
   }
