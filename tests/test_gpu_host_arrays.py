@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n,nrhs,pad", [(1, 1, 3), (7, 5, 1), (130, 1, 70), (500, 4, 12), (2100, 3, 5)])
 def test_strided_columns(dev, n, nrhs, pad):
     a, b = la.matrix(2, n, n, n), la.matrix(2, n + 1, n, nrhs)
-    a0, b0, p0 = np.asfortranarray(a), np.asfortranarray(b), np.zeros(n, np.int32)
+    a0, b0, p0 = a.copy(order="F"), b.copy(order="F"), np.zeros(n, np.int32)
     assert la.dgesv(n, nrhs, a0, n, p0, b0, n) == 0
     lda, ldb = n + pad, n + 2 * pad
     a1, b1 = np.full((lda, n), 3.5, order="F"), np.full((ldb, nrhs), 4.5, order="F")
