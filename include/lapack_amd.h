@@ -230,9 +230,10 @@ int lapack_amd_dgesv_adjoint_async(int n, int nrhs, const double* d_lu, int lda,
  *
  * A plan fixes the orders (host array n[batch]) and the precision ('d' or
  * 's'), orders the matrices by decreasing n for the persistent launch, and
- * -- with autotune != 0 -- times the kernel configurations (panel width NB,
- * workgroup size) on synthetic matrices of the plan's sizes and keeps the
- * fastest.  Creating a plan allocates; the *_batched_async launches do
+ * -- for orders past 512, with autotune != 0 -- times the kernel
+ * configurations (panel width NB, workgroup size) on synthetic matrices of the
+ * plan's sizes and keeps the fastest; up to 512 it takes the configuration
+ * (32, 512), which needs no trial.  Creating a plan allocates; the *_batched_async launches do
  * not, and may be captured in a hipGraph and replayed. */
 typedef struct lapack_amd_batch_plan lapack_amd_batch_plan;
 int lapack_amd_batch_plan_create(lapack_amd_batch_plan** plan, int batch, const int* n, char precision,

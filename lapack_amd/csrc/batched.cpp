@@ -8,7 +8,8 @@
 // nothing and make only kernel launches, so they can be captured in a
 // hipGraph and replayed.
 //
-// Autotuner: for each configuration that fits the device's LDS at the
+// Orders up to 512 take the register form (batched_leaf.hip).  Above, the
+// autotuner: for each configuration that fits the device's LDS at the
 // batch's largest n, the plan's own size distribution is factored on
 // synthetic uniform(-1,1) matrices (a deterministic sample of up to 2048 of
 // the batch's sizes) and timed with HIP events; the fastest is kept, and
@@ -40,18 +41,23 @@ std::map<std::tuple<int, int, int>, int> g_tuned;  // (elem, nmax, mean n / 16) 
 }  // namespace
 }  // namespace la
 
+// The register form of the factorization (batched_leaf.hip), as one more
+// configuration: 32 columns a block, up to 512 threads a workgroup.
+constexpr int LEAF_CFG = 1000, LEAF_NB = 32, LEAF_NT = 512;
+
 struct lapack_amd_batch_plan {
   int batch = 0;
   int nmax = 0;
   int elem = 8;     // 8: FP64, 4: FP32
-  int cfg = -1;     // kernel configuration index
+  int cfg = -1;     // kernel configuration index; LEAF_CFG: the register form
+  la::BatchedLeafPlan leaf;  // ranges and grids of the register form
   int grid_f = 1;   // persistent grid of the getrf launch
   int grid_s = 1;   // persistent grid of the getrs launch
   int grid_t = 1;   // persistent grid of the adjoint's transposed solve (FP64)
   int dev = -1;
   int* d_n = nullptr;
   int* d_order = nullptr;
-  unsigned* d_counter = nullptr;  // [0] getrf, [1] getrs, [2] adjoint
+  unsigned* d_counter = nullptr;  // [0] getrf, [1] getrs, [2] adjoint, [4..7] the register form's ranges
   std::vector<int> n;
   double tuned_ms = 0.0;
 };
@@ -146,7 +152,15 @@ int tune_plan(lapack_amd_batch_plan* p, hipStream_t s) {
   return 0;
 }
 
+// Orders up to 512 take the register form, without a trial: it was faster than
+// the best of the panel forms for every batch measured.  Uniform orders,
+// best panel form -> register form, us:  FP64: 8 of 4..12 43 -> 33, 2000 of
+// 4..12 71 -> 64, 1000 of 16..64 197 -> 103, 3000 of 8..160 1233 -> 893, 4 of
+// 300..512 3447 -> 1797, 300 of 400..512 5977 -> 3714, 1000 of 100..256 1666 ->
+// 1472, 10000 of 16..512 62967 -> 32616.  FP32: 43 -> 31, 72 -> 68, 189 -> 118,
+// 983 -> 695, 3202 -> 1354, 5059 -> 1837, 1481 -> 858.
 int default_cfg(int nmax, int elem) {
+  if (nmax <= batched_leaf_nmax()) return LEAF_CFG;
   // Largest panel that fits, 256 threads (autotuning usually confirms NB 16 or 32).
   for (int cfg : {3, 1, 0, 5})
     if (batched_getrf_smem(cfg, nmax, elem) <= (size_t)lds_limit()) return cfg;
@@ -161,7 +175,13 @@ using namespace la;
 // Persistent grids for the plan's configuration (queries the runtime once).
 static int rc_grid(lapack_amd_batch_plan* p) {
   const int nm = std::max(p->nmax, 1), b = std::max(p->batch, 1);
-  const int gf = p->elem == 8 ? batched_getrf_grid<double>(p->cfg, b, nm) : batched_getrf_grid<float>(p->cfg, b, nm);
+  if (p->cfg == LEAF_CFG) {
+    std::vector<int> sorted = p->n;
+    std::sort(sorted.begin(), sorted.end(), std::greater<int>());
+    if (p->elem == 8) batched_leaf_plan<double>(p->batch, sorted.data(), &p->leaf);
+    else batched_leaf_plan<float>(p->batch, sorted.data(), &p->leaf);
+  }
+  const int gf = p->cfg == LEAF_CFG ? 1 : p->elem == 8 ? batched_getrf_grid<double>(p->cfg, b, nm) : batched_getrf_grid<float>(p->cfg, b, nm);
   const int gs = p->elem == 8 ? batched_getrs_grid<double>(b, nm) : batched_getrs_grid<float>(b, nm);
   if (gf < 0) return gf;
   if (gs < 0) return gs;
@@ -209,7 +229,7 @@ int lapack_amd_batch_plan_create(lapack_amd_batch_plan** out, int batch, const i
   }
   p->cfg = default_cfg(std::max(p->nmax, 1), p->elem);
   if (p->cfg < 0) { lapack_amd_batch_plan_destroy(p); return LA_ERR_LIMIT; }
-  if (autotune && batch > 0) {
+  if (autotune && batch > 0 && p->cfg != LEAF_CFG) {
     long long sum = 0;
     for (int v : p->n) sum += v;
     const auto key = std::make_tuple(p->elem, p->nmax, (int)(sum / batch / 16));
@@ -253,8 +273,8 @@ void lapack_amd_batch_plan_destroy(lapack_amd_batch_plan* p) {
 
 int lapack_amd_batch_plan_config(const lapack_amd_batch_plan* p, int* nb, int* nthreads, double* tuned_ms) {
   if (!p) return -1;
-  int b = 0, t = 0;
-  batched_getrf_config(p->cfg, &b, &t);
+  int b = LEAF_NB, t = LEAF_NT;
+  if (p->cfg != LEAF_CFG) batched_getrf_config(p->cfg, &b, &t);
   if (nb) *nb = b;
   if (nthreads) *nthreads = t;
   if (tuned_ms) *tuned_ms = p->tuned_ms;
@@ -263,6 +283,10 @@ int lapack_amd_batch_plan_config(const lapack_amd_batch_plan* p, int* nb, int* n
 
 int lapack_amd_batch_plan_set_config(lapack_amd_batch_plan* p, int nb, int nthreads) {
   if (!p) return -1;
+  if (nb == LEAF_NB && nthreads == LEAF_NT && std::max(p->nmax, 1) <= batched_leaf_nmax()) {
+    p->cfg = LEAF_CFG;
+    return rc_grid(p);
+  }
   for (int c = 0; c < batched_getrf_configs(); ++c) {
     int b, t;
     batched_getrf_config(c, &b, &t);
@@ -283,7 +307,10 @@ int lapack_amd_dgetrf_batched_async(const lapack_amd_batch_plan* p, double* cons
   if (!p) return -1;
   if (p->elem != 8) return -1;
   if (p->batch == 0) return 0;
-  int rc = launch_getrf_batched<double>(p->cfg, p->grid_f, p->batch, p->nmax, p->d_n, d_a, d_lda, d_ipiv, d_info,
+  int rc = p->cfg == LEAF_CFG
+               ? launch_getrf_batched_leaf<double>(p->leaf, p->d_n, d_a, d_lda, d_ipiv, d_info, p->d_order,
+                                                p->d_counter + 4, (hipStream_t)stream)
+               : launch_getrf_batched<double>(p->cfg, p->grid_f, p->batch, p->nmax, p->d_n, d_a, d_lda, d_ipiv, d_info,
                                         p->d_order,
                                         p->d_counter, (hipStream_t)stream);
   return rc ? rc : hipc(hipGetLastError());
@@ -293,7 +320,10 @@ int lapack_amd_sgetrf_batched_async(const lapack_amd_batch_plan* p, float* const
   if (!p) return -1;
   if (p->elem != 4) return -1;
   if (p->batch == 0) return 0;
-  int rc = launch_getrf_batched<float>(p->cfg, p->grid_f, p->batch, p->nmax, p->d_n, d_a, d_lda, d_ipiv, d_info,
+  int rc = p->cfg == LEAF_CFG
+               ? launch_getrf_batched_leaf<float>(p->leaf, p->d_n, d_a, d_lda, d_ipiv, d_info, p->d_order,
+                                                p->d_counter + 4, (hipStream_t)stream)
+               : launch_getrf_batched<float>(p->cfg, p->grid_f, p->batch, p->nmax, p->d_n, d_a, d_lda, d_ipiv, d_info,
                                        p->d_order,
                                        p->d_counter, (hipStream_t)stream);
   return rc ? rc : hipc(hipGetLastError());

@@ -11,7 +11,9 @@
 // the tail of the launch short), so the grid drains when the counter passes
 // the batch size; every loop is bounded by the matrix order.
 //
-// DGETRF per matrix, right-looking and blocked with panel width NB:
+// DGETRF per matrix (orders past 512 and configurations that a caller selects;
+// batched_leaf.hip holds the form for smaller ones), right-looking and blocked
+// with panel width NB:
 //   1. the panel A(k0:n, k0:k0+w) is loaded into LDS and factored there
 //      column by column: IDAMAX (BLAS/SRC/idamax.f:93-122) by wavefront
 //      reductions over 64-bit keys that order like its rule (first max,

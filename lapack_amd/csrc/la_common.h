@@ -194,6 +194,18 @@ int launch_adjoint_batched(int grid, int batch, int nmax, const int* nv, const i
                            double* const* xbv, const int* ldxbv, double* const* abv, const int* ldabv,
                            int accumulate, const int* order, unsigned* counter, hipStream_t s);
 
+// The batch's LU for orders up to batched_leaf_nmax() (batched_leaf.hip):
+// ranges of the decreasing order, one persistent launch each; counters: four
+// device words the launcher zeroes.
+struct BatchedLeafPlan {
+  int first[4], last[4], grid[4];
+};
+int batched_leaf_nmax();
+template <class T> void batched_leaf_plan(int batch, const int* sorted, BatchedLeafPlan* p);
+template <class T>
+int launch_getrf_batched_leaf(const BatchedLeafPlan& p, const int* nv, T* const* av, const int* ldav, int* const* ipv,
+                              int* infov, const int* order, unsigned* counters, hipStream_t s);
+
 // Triangular sweeps of DGETRS in one launch each (getrs.hip).  which: 0 = L
 // (unit lower), 1 = U, 2 = U^T, 3 = L^T; the right-hand sides Xin (n x nrhs,
 // ldxi) are read, the solution written to X (ldx; a different buffer, whose

@@ -24,7 +24,7 @@
 // Bound by latency for the few columns on the panel's path (a block: 64
 // dependent steps), by the matrix cores and the triangle's re-reads from L2
 // for all columns of a large matrix.
-#include "la_common.h"
+#include "leaf.h"
 
 namespace la {
 namespace {
@@ -44,21 +44,6 @@ template <> struct SMfma<float> {
   }
   static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
 };
-
-// acc += (x of lane 16*(lane/16) + KS) * l; every lane active.  The s_nop
-// covers the wait states a DPP source needs after a vector write of it.
-template <int KS>
-__device__ __forceinline__ void fmac_from(double& acc, double x, double l) {
-  asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc)
-      : "v"(x), "v"(l), "n"(KS));
-}
-template <int KS>
-__device__ __forceinline__ void fmac_from(float& acc, float x, float l) {
-  asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc)
-      : "v"(x), "v"(l), "n"(KS));
-}
 
 constexpr int SB = 64;        // rows of a solve block
 constexpr int SC = 16;        // columns of A a workgroup owns
