@@ -52,8 +52,9 @@ struct lapack_amd_batch_plan {
   int cfg = -1;     // kernel configuration index; LEAF_CFG: the register form
   la::BatchedLeafPlan leaf;  // ranges and grids of the register form
   int grid_f = 1;   // persistent grid of the getrf launch
-  int grid_s = 1;   // persistent grid of the getrs launch
-  int grid_t = 1;   // persistent grid of the adjoint's transposed solve (FP64)
+  la::BatchedSolvePlan solve;    // the getrs launches
+  la::BatchedSolvePlan solve_t;  // the adjoint's transposed solve (FP64)
+  bool adjoint = false;          // its right-hand sides fit in LDS
   int dev = -1;
   int* d_n = nullptr;
   int* d_order = nullptr;
@@ -180,16 +181,17 @@ static int rc_grid(lapack_amd_batch_plan* p) {
     std::sort(sorted.begin(), sorted.end(), std::greater<int>());
     if (p->elem == 8) batched_leaf_plan<double>(p->batch, sorted.data(), &p->leaf);
     else batched_leaf_plan<float>(p->batch, sorted.data(), &p->leaf);
+  } else {
+    const int gf = p->elem == 8 ? batched_getrf_grid<double>(p->cfg, b, nm) : batched_getrf_grid<float>(p->cfg, b, nm);
+    if (gf < 0) return gf;
+    p->grid_f = gf;
   }
-  const int gf = p->cfg == LEAF_CFG ? 1 : p->elem == 8 ? batched_getrf_grid<double>(p->cfg, b, nm) : batched_getrf_grid<float>(p->cfg, b, nm);
-  const int gs = p->elem == 8 ? batched_getrs_grid<double>(b, nm) : batched_getrs_grid<float>(b, nm);
-  if (gf < 0) return gf;
-  if (gs < 0) return gs;
-  p->grid_f = gf;
-  p->grid_s = gs;
-  // the adjoint's grid; a plan whose orders exceed its LDS keeps 0 (the
-  // adjoint then reports LA_ERR_LIMIT)
-  p->grid_t = p->elem == 8 ? std::max(0, batched_getrs_t_grid<double>(b, nm)) : 0;
+  const int rs = p->elem == 8 ? batched_solve_plan<double, false>(b, nm, &p->solve)
+                              : batched_solve_plan<float, false>(b, nm, &p->solve);
+  if (rs < 0) return rs;
+  // a plan whose orders exceed the transposed solve's LDS makes the adjoint
+  // report LA_ERR_LIMIT
+  p->adjoint = p->elem == 8 && batched_solve_plan<double, true>(b, nm, &p->solve_t) == 0;
   return 0;
 }
 
@@ -334,7 +336,7 @@ int lapack_amd_dgetrs_batched_async(const lapack_amd_batch_plan* p, const int* d
   if (!p) return -1;
   if (p->elem != 8) return -1;
   if (p->batch == 0) return 0;
-  int rc = launch_getrs_batched<double>(p->grid_s, p->batch, p->nmax, p->d_n, d_nrhs, d_a, d_lda, d_ipiv, d_b, d_ldb,
+  int rc = launch_getrs_batched<double>(p->solve, p->batch, p->nmax, p->d_n, d_nrhs, d_a, d_lda, d_ipiv, d_b, d_ldb,
                                         p->d_order, p->d_counter + 1, (hipStream_t)stream);
   return rc ? rc : hipc(hipGetLastError());
 }
@@ -344,7 +346,7 @@ int lapack_amd_sgetrs_batched_async(const lapack_amd_batch_plan* p, const int* d
   if (!p) return -1;
   if (p->elem != 4) return -1;
   if (p->batch == 0) return 0;
-  int rc = launch_getrs_batched<float>(p->grid_s, p->batch, p->nmax, p->d_n, d_nrhs, d_a, d_lda, d_ipiv, d_b, d_ldb,
+  int rc = launch_getrs_batched<float>(p->solve, p->batch, p->nmax, p->d_n, d_nrhs, d_a, d_lda, d_ipiv, d_b, d_ldb,
                                        p->d_order, p->d_counter + 1, (hipStream_t)stream);
   return rc ? rc : hipc(hipGetLastError());
 }
@@ -358,8 +360,8 @@ int lapack_amd_dgesv_adjoint_batched_async(const lapack_amd_batch_plan* p, const
   if (!p) return -1;
   if (p->elem != 8) return -1;
   if (p->batch == 0) return 0;
-  if (p->grid_t <= 0) return LA_ERR_LIMIT;
-  int rc = launch_adjoint_batched(p->grid_t, p->batch, p->nmax, p->d_n, d_nrhs, d_lu, d_lda, d_ipiv, d_x, d_ldx,
+  if (!p->adjoint) return LA_ERR_LIMIT;
+  int rc = launch_adjoint_batched(p->solve_t, p->batch, p->nmax, p->d_n, d_nrhs, d_lu, d_lda, d_ipiv, d_x, d_ldx,
                                   d_xbar, d_ldxbar, d_abar, d_ldabar, accumulate, p->d_order, p->d_counter + 2,
                                   (hipStream_t)stream);
   return rc ? rc : hipc(hipGetLastError());

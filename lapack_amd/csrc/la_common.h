@@ -180,19 +180,24 @@ size_t batched_getrf_smem(int idx, int nmax, int elem);
 // grid: workgroups of the persistent launch (batched_*_grid, computed once
 // per plan so that the launches themselves make no runtime queries).
 template <class T> int batched_getrf_grid(int cfg, int batch, int nmax);
-template <class T> int batched_getrs_grid(int batch, int nmax);
 template <class T>
 int launch_getrf_batched(int cfg, int grid, int batch, int nmax, const int* nv, T* const* av, const int* ldav,
                          int* const* ipv, int* infov, const int* order, unsigned* counter, hipStream_t s);
+// The batch's triangular solves (batched_solve.hip): workgroups of 16 waves
+// (wide) or 4; counter: a device word the launcher zeroes.
+struct BatchedSolvePlan {
+  bool wide = false;
+  int grid = 1;
+};
+template <class T, bool TRANS> int batched_solve_plan(int batch, int nmax, BatchedSolvePlan* p);
 template <class T>
-int launch_getrs_batched(int grid, int batch, int nmax, const int* nv, const int* nrhsv, T* const* av,
+int launch_getrs_batched(const BatchedSolvePlan& p, int batch, int nmax, const int* nv, const int* nrhsv, T* const* av,
                          const int* ldav, int* const* ipv, T* const* bv, const int* ldbv, const int* order,
                          unsigned* counter, hipStream_t s);
-template <class T> int batched_getrs_t_grid(int batch, int nmax);
-int launch_adjoint_batched(int grid, int batch, int nmax, const int* nv, const int* nrhsv, double* const* luv,
-                           const int* ldluv, int* const* ipv, double* const* xv, const int* ldxv,
-                           double* const* xbv, const int* ldxbv, double* const* abv, const int* ldabv,
-                           int accumulate, const int* order, unsigned* counter, hipStream_t s);
+int launch_adjoint_batched(const BatchedSolvePlan& p, int batch, int nmax, const int* nv, const int* nrhsv,
+                           double* const* luv, const int* ldluv, int* const* ipv, double* const* xv, const int* ldxv,
+                           double* const* xbv, const int* ldxbv, double* const* abv, const int* ldabv, int accumulate,
+                           const int* order, unsigned* counter, hipStream_t s);
 
 // The batch's LU for orders up to batched_leaf_nmax() (batched_leaf.hip):
 // ranges of the decreasing order, one persistent launch each; counters: four
