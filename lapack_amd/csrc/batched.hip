@@ -27,6 +27,7 @@
 //      with its zero test), staged in LDS, then the update A22 -= A21*U12
 //      (dgetrf.f:212-216) in 4x4 register tiles.
 #include "la_common.h"
+#include "mfma.h"
 
 namespace la {
 namespace {
@@ -52,25 +53,6 @@ __device__ __forceinline__ void wave_argmax(u64& key, int& row) {
     if (k2 > key || (k2 == key && r2 < row)) { key = k2; row = r2; }
   }
 }
-
-// FP64 / FP32 16x16x4 matrix-core product on gfx950: lane l holds A(l%16,
-// l/16) and B(l/16, l%16) of a k-step; accumulator register r of lane l
-// holds D(row(l/16, r), l%16).
-template <class T> struct BMfma;
-template <> struct BMfma<double> {
-  typedef la_d4 acc_t;
-  static __device__ __forceinline__ acc_t op(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return lk + 4 * r; }
-};
-template <> struct BMfma<float> {
-  typedef la_f4 acc_t;
-  static __device__ __forceinline__ acc_t op(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
-};
 
 constexpr int TM = 4, TN = 4, TX = 16;
 
@@ -292,7 +274,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NB <= 16 ? 2
         // l%16 walks rows and C moves in whole 128-byte pieces; C is loaded
         // before the products.
         {
-          typedef BMfma<T> MM;
+          typedef Mfma<T> MM;
           typedef typename MM::acc_t acc_t;
           const int lane = tid & 63, wave = tid >> 6;
           const int li = lane & 15, lk = lane >> 4;

@@ -28,27 +28,12 @@
 // the trailing matrix read and written once per 32 columns (n^3/6 bytes per
 // matrix in FP64) where the batch exceeds the caches.
 #include "leaf.h"
+#include "mfma.h"
 
 #include <algorithm>
 
 namespace la {
 namespace {
-
-template <class T> struct LMfma;
-template <> struct LMfma<double> {
-  typedef la_d4 acc_t;
-  static __device__ __forceinline__ acc_t op(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return lk + 4 * r; }
-};
-template <> struct LMfma<float> {
-  typedef la_f4 acc_t;
-  static __device__ __forceinline__ acc_t op(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
-};
 
 constexpr int BW = 32;  // columns of a block
 
@@ -78,7 +63,7 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4))) void g
                                                                     int* __restrict__ infov,
                                                                     const int* __restrict__ order,
                                                                     unsigned* counter) {
-  typedef LMfma<T> MM;
+  typedef Mfma<T> MM;
   typedef typename MM::acc_t acc_t;
   constexpr int NW = NTH / 64;
   constexpr int CB = NTH >= 256 ? 64 : NTH >= 128 ? 32 : 16;  // columns of a pass's piece

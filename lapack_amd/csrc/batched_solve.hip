@@ -30,34 +30,19 @@
 // 64-step substitutions by shuffles and interchanges by one lane: 10000 solves
 // of order 16..512 4700 -> 1720 us, the 256 adjoints 6420 -> 1174 (650 of them
 // the solve: 3.3 TB/s of A; floor of both halves 930).
-#include "leaf.h"
+#include "tri_block.h"
+#include "mfma.h"
 
 #include <algorithm>
 
 namespace la {
 namespace {
 
-template <class T> struct SMfma;
-template <> struct SMfma<double> {
-  typedef la_d4 acc_t;
-  static __device__ __forceinline__ acc_t op(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return lk + 4 * r; }
-};
-template <> struct SMfma<float> {
-  typedef la_f4 acc_t;
-  static __device__ __forceinline__ acc_t op(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
-};
-
 // Groups of waves that share a block's product (4 waves: 16 rows each).
 template <int NT> constexpr int groups() { return NT / 256; }
 
 template <class T, int NT, int NR> struct SolveLds {
-  T tri[10][16][17];  // sub-block (mi >= mk) at mi (mi + 1) / 2 + mk: -coefficient [k][i]
+  TriBlock<T> tri;
   T dia[64], rec[64];
   T red[groups<NT>()][groups<NT>() > 1 ? NR : 1][64];
   int item;
@@ -67,32 +52,10 @@ template <class T, int NT, int NR> struct SolveLds {
 // keeps the rows that op(A) = A^T takes apart in the banks; 4 more, A's.)
 inline int solve_ldx(int nmax, bool trans) { return (nmax + 63) / 64 * 64 + (trans ? 1 : 4); }
 
-template <class T>
-__device__ __forceinline__ T div_by(T t, T d, T r) {
-  const T q = t * r;
-  return fma(fma(-q, d, t), r, q);
-}
-
-// Step K of the substitution in sub-block KM (rows 16 KM .. + 15 in x[KM] of 16 lanes).
-template <class T, bool UNIT, int KM, int KS>
-__device__ __forceinline__ void sub_step(T (&x)[4], const T (&d)[4], const T (&r)[4], const T (*tri)[16][17], int sub) {
-  if constexpr (KS < 16) {
-    T q = x[KM];
-    if constexpr (!UNIT) q = div_by(q, d[KM], r[KM]);
-    const T* c = &tri[KM * (KM + 1) / 2 + KM][KS][sub];
-    fmac_from<KS>(x[KM], q, *c);
-#pragma unroll
-    for (int m = KM + 1; m < 4; ++m) fmac_from<KS>(x[m], q, tri[m * (m + 1) / 2 + KM][KS][sub]);
-    sub_step<T, UNIT, KM, KS + 1>(x, d, r, tri, sub);
-  } else if constexpr (!UNIT) {
-    x[KM] = div_by(x[KM], d[KM], r[KM]);
-  }
-}
-
 // One sweep: FWD rows 0, 1, ..; otherwise rows n-1, n-2, ..
 template <class T, bool TRANS, bool FWD, bool UNIT, int NT, int NR>
 __device__ __forceinline__ void sweep(const T* A, long lda, int n, T* X, int ldx, int nr, SolveLds<T, NT, NR>& S) {
-  typedef SMfma<T> MM;
+  typedef Mfma<T> MM;
   typedef typename MM::acc_t acc_t;
   constexpr int G = groups<NT>();
   constexpr int SU = (10 + G - 1) / G;  // a thread's sub-blocks of the triangle, an element of each
@@ -166,7 +129,7 @@ __device__ __forceinline__ void sweep(const T* A, long lda, int n, T* X, int ldx
 #pragma unroll
     for (int u = 0; u < SU; ++u) {
       const int sb = tid / 256 + G * u;
-      if (sb < 10) S.tri[sb][TRANS ? ta : tc][TRANS ? tc : ta] = -t[u];
+      if (sb < 10) S.tri.c[sb][TRANS ? ta : tc][TRANS ? tc : ta] = -t[u];
     }
     if (!UNIT && tid < 64) {
       S.dia[tid] = dg;
@@ -193,10 +156,7 @@ __device__ __forceinline__ void sweep(const T* A, long lda, int n, T* X, int ldx
         d[m] = UNIT ? T(1) : S.dia[i];
         r[m] = UNIT ? T(1) : S.rec[i];
       }
-      if (m_lo <= 0 && m_hi > 0) sub_step<T, UNIT, 0, 0>(x, d, r, S.tri, li);
-      if (m_lo <= 1 && m_hi > 1) sub_step<T, UNIT, 1, 0>(x, d, r, S.tri, li);
-      if (m_lo <= 2 && m_hi > 2) sub_step<T, UNIT, 2, 0>(x, d, r, S.tri, li);
-      if (m_lo <= 3 && m_hi > 3) sub_step<T, UNIT, 3, 0>(x, d, r, S.tri, li);
+      tri_solve<T, UNIT ? DIAG_UNIT : DIAG_DIVIDE>(x, d, r, S.tri, li, m_lo, m_hi);
 #pragma unroll
       for (int m = 0; m < 4; ++m)
         if (q < nr) X[row_of(16 * m + li) + q * ldx] = x[m];

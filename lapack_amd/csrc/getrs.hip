@@ -1,4 +1,5 @@
-// getrs.hip -- the triangular solves of DGETRS as one launch per sweep.
+// getrs.hip -- the triangular solves of DGETRS as one launch per sweep, for two
+// and more right-hand sides (tri_line.hip has the sweep for one).
 //
 // DGETRS (SRC/dgetrs.f:181-218) solves with L (unit lower) then U (upper),
 // or U^T then L^T for 'T'.  Each sweep is M x = y for one triangular M =
@@ -29,7 +30,8 @@
 // Every wait is bounded; one that gives up sets *err, and the other waits
 // poll *err and give up as well, so every workgroup runs to its end (the
 // caller then leaves B as it was and reports the failure).
-#include "la_common.h"
+#include "mfma.h"
+#include "tri_block.h"
 
 #include <algorithm>
 
@@ -90,49 +92,7 @@ __device__ void invert_diag(T (*sD)[TB + 1], T* tmp) {
   }
 }
 
-// The sentinel that marks a value of x not yet written: a quiet NaN with a
-// fixed payload.  A computed value with exactly these bits (only a NaN
-// carrying this payload from the input) is stored as the NaN `alt` instead.
-template <class T> struct Sent;
-template <> struct Sent<double> {
-  using U = unsigned long long;
-  static constexpr U bits = 0x7FFC00005E471E57ull, alt = 0x7FFC00005E471E56ull;
-};
-template <> struct Sent<float> {
-  using U = unsigned;
-  static constexpr U bits = 0x7FC5E471u, alt = 0x7FC5E470u;
-};
-template <class T>
-__device__ __forceinline__ bool is_sent(T v) {
-  return __builtin_bit_cast(typename Sent<T>::U, v) == Sent<T>::bits;
-}
-template <class T>
-__device__ __forceinline__ T canon(T v) {
-  return is_sent(v) ? __builtin_bit_cast(T, Sent<T>::alt) : v;
-}
-
-constexpr unsigned SPIN_LIMIT = 1u << 22;
-
-// FP64 / FP32 16x16x4 matrix-core product on gfx950: lane l holds A(l%16,
-// l/16) and B(l/16, l%16) of a k-step; accumulator register r of lane l
-// holds D(row(l/16, r), l%16).
-template <class T> struct TriMfma;
-template <> struct TriMfma<double> {
-  typedef la_d4 acc_t;
-  static __device__ __forceinline__ acc_t op(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return lk + 4 * r; }
-};
-template <> struct TriMfma<float> {
-  typedef la_f4 acc_t;
-  static __device__ __forceinline__ acc_t op(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
-};
-
-// QN: right-hand sides handled per launch (1, 4 or 16).  Reads the
+// QN: right-hand sides handled per launch (4 or 16).  Reads the
 // right-hand sides from Xin, writes x to X (filled with the sentinel
 // beforehand; the two may not overlap).
 template <class T, int QN, bool LOWERM, bool UNIT, bool TRANS>
@@ -142,7 +102,7 @@ __global__ __launch_bounds__(256) void tri_chain_kernel(int n, int nrhs, const T
   // MF: 16 right-hand sides, products on the matrix cores, wave g owning
   // rows 16g .. 16g+15 of the block; otherwise products on the vector units
   constexpr bool MF = QN == 16;
-  typedef TriMfma<T> MM;
+  typedef Mfma<T> MM;
   typedef typename MM::acc_t acc_t;
   constexpr int XS = QN + 1;  // row stride of the [row][rhs] stagings
   constexpr int NBUF_MF = DEPB * TB * XS;
@@ -489,7 +449,7 @@ void launch_chain(int n, int nrhs, const T* A, long lda, const T* Xin, long ldxi
     const T* Xi = Xin + (long)q0 * ldxi;
     T* Xq = X + (long)q0 * ldx;
     unsigned* tk = ctl + sl;
-    if (nq == 1) launch_chain_q<T, 1, LOWERM, UNIT, TRANS>(nblk, n, nq, A, lda, Xi, ldxi, Xq, ldx, tk, err, s);
+    if (nq == 1) launch_tri_line<T>(TRANS ? (LOWERM ? 2 : 3) : (LOWERM ? 0 : 1), n, A, lda, Xi, Xq, tk, err, s);
     else if (nq <= 4) launch_chain_q<T, 4, LOWERM, UNIT, TRANS>(nblk, n, nq, A, lda, Xi, ldxi, Xq, ldx, tk, err, s);
     else launch_chain_q<T, 16, LOWERM, UNIT, TRANS>(nblk, n, nq, A, lda, Xi, ldxi, Xq, ldx, tk, err, s);
   }

@@ -211,6 +211,11 @@ template <class T>
 int launch_getrf_batched_leaf(const BatchedLeafPlan& p, const int* nv, T* const* av, const int* ldav, int* const* ipv,
                               int* infov, const int* order, unsigned* counters, hipStream_t s);
 
+// One right-hand side (tri_line.hip).
+template <class T>
+void launch_tri_line(int which, int n, const T* A, long lda, const T* Xin, T* X, unsigned* ticket, int* err,
+                     hipStream_t s);
+
 // Triangular sweeps of DGETRS in one launch each (getrs.hip).  which: 0 = L
 // (unit lower), 1 = U, 2 = U^T, 3 = L^T; the right-hand sides Xin (n x nrhs,
 // ldxi) are read, the solution written to X (ldx; a different buffer, whose

@@ -1,0 +1,82 @@
+// tri_block.h -- what the triangular sweeps share: the substitution with a 64 x
+// 64 triangle laid out in LDS in its own order, 16 lanes a right-hand side, and
+// the sentinel of values of x that are still to come.
+#pragma once
+#include "leaf.h"
+
+namespace la {
+
+// The coefficients below the diagonal by 16 x 16 sub-blocks: sub-block
+// (mi >= mk) at mi (mi + 1) / 2 + mk holds -M(16 mi + i, 16 mk + k) at [k][i], zero
+// for i <= k of the diagonal ones.
+template <class T> struct TriBlock {
+  T c[10][16][17];
+};
+
+// t / d from r = 1 / d: the product corrected by its remainder, which rounds
+// like the division while d and t / d are normal numbers.
+template <class T>
+__device__ __forceinline__ T div_by(T t, T d, T r) {
+  const T q = t * r;
+  return fma(fma(-q, d, t), r, q);
+}
+
+enum Diag { DIAG_UNIT, DIAG_DIVIDE, DIAG_MULTIPLY };
+
+template <class T, Diag D>
+__device__ __forceinline__ T by_diag(T x, T d, T r) {
+  if constexpr (D == DIAG_DIVIDE) return div_by(x, d, r);
+  else if constexpr (D == DIAG_MULTIPLY) return x * r;
+  else return x;
+}
+
+// Steps KS .. 15 of sub-block KM; lane sub of 16 holds rows 16 m + sub in x[m],
+// with their diagonals d and reciprocals r.  Per step one DPP product a
+// sub-block still to come, the first of them the chain (about 16 cycles).
+template <class T, Diag D, int KM, int KS>
+__device__ __forceinline__ void tri_step(T (&x)[4], const T (&d)[4], const T (&r)[4], const TriBlock<T>& tri, int sub) {
+  if constexpr (KS < 16) {
+    if constexpr (KS % 8 == 0) asm volatile("" ::: "memory");  // (coefficients of 8 steps in flight, not of all)
+    const T q = by_diag<T, D>(x[KM], d[KM], r[KM]);
+#pragma unroll
+    for (int m = KM; m < 4; ++m) fmac_from<KS>(x[m], q, tri.c[m * (m + 1) / 2 + KM][KS][sub]);
+    tri_step<T, D, KM, KS + 1>(x, d, r, tri, sub);
+  } else {
+    x[KM] = by_diag<T, D>(x[KM], d[KM], r[KM]);
+  }
+}
+
+// Sub-blocks m_lo .. m_hi - 1 (the others hold rows past the matrix).
+template <class T, Diag D>
+__device__ __forceinline__ void tri_solve(T (&x)[4], const T (&d)[4], const T (&r)[4], const TriBlock<T>& tri, int sub,
+                                          int m_lo, int m_hi) {
+  if (m_lo <= 0 && m_hi > 0) tri_step<T, D, 0, 0>(x, d, r, tri, sub);
+  if (m_lo <= 1 && m_hi > 1) tri_step<T, D, 1, 0>(x, d, r, tri, sub);
+  if (m_lo <= 2 && m_hi > 2) tri_step<T, D, 2, 0>(x, d, r, tri, sub);
+  if (m_lo <= 3 && m_hi > 3) tri_step<T, D, 3, 0>(x, d, r, tri, sub);
+}
+
+// The sentinel that marks a value of x not yet written: a quiet NaN with a
+// fixed payload.  A computed value with exactly these bits (only a NaN
+// carrying this payload from the input) is stored as the NaN `alt` instead.
+template <class T> struct Sent;
+template <> struct Sent<double> {
+  using U = unsigned long long;
+  static constexpr U bits = 0x7FFC00005E471E57ull, alt = 0x7FFC00005E471E56ull;
+};
+template <> struct Sent<float> {
+  using U = unsigned;
+  static constexpr U bits = 0x7FC5E471u, alt = 0x7FC5E470u;
+};
+template <class T>
+__device__ __forceinline__ bool is_sent(T v) {
+  return __builtin_bit_cast(typename Sent<T>::U, v) == Sent<T>::bits;
+}
+template <class T>
+__device__ __forceinline__ T canon(T v) {
+  return is_sent(v) ? __builtin_bit_cast(T, Sent<T>::alt) : v;
+}
+
+constexpr unsigned SPIN_LIMIT = 1u << 22;
+
+}  // namespace la

@@ -1,0 +1,340 @@
+// tri_line.hip -- one right-hand side through a triangle: a sweep of DGETRS
+// (SRC/dgetrs.f:181-218) as one launch.
+//
+// M x = y for triangular M = op(tri(A)).  A sweep reads the triangle once and is
+// a chain through its diagonal blocks; every link of the chain between two
+// workgroups costs a store to memory and a load from it (1 us and more across
+// XCDs), so a block is as large as a workgroup can finish in about that time:
+//   * one workgroup of 16 waves per 128 rows of x, ordered by a ticket taken at
+//     the start: a workgroup waits only for blocks of lower tickets, which are
+//     running, so every wait ends;
+//   * each wave owns 1024 elements of every 128 x 128 tile of M that the block
+//     depends on, reads them a tile ahead, polls the values of x it needs itself
+//     (the sentinel says which are not there yet) and multiplies: no barrier
+//     until the last tile is done;
+//   * before the first tile both 64-row diagonal triangles are inverted, 16 x 16
+//     blocks by substitution and the rest by products with them, and kept, with
+//     the tile between them, in registers: 4 elements a thread, a row on 16
+//     lanes.  After the last tile the two halves are a product each, and one
+//     between them.
+// Sums: 16 products of a tile, then one term per tile, then 8 parts.
+// Bound: at n = 6001 a link takes 3.5 us (M = L, U) or 4.5 (transposed): reading a
+// tile of 128 KB at what one CU gets from memory, 30 to 50 GB/s; 1.4 of it the
+// way of x through memory.  64-row blocks of 4 waves with a round's x in LDS took
+// 2.5 to 6.4 us for half the rows.  n = 6001, one right-hand side, FP64, with
+// the permutation: 'N' 541 -> 396 us, 'T' 978 -> 490; n = 100 84 -> 66.
+// Every wait is bounded; one that gives up sets *err, and the others poll *err
+// and give up as well, so every workgroup runs to its end.
+#include "tri_block.h"
+#include "mfma.h"
+
+namespace la {
+namespace {
+
+constexpr int RB = 128;  // rows of a block
+
+// Two (FP64) or four consecutive values with the alignment of one.
+template <class T> struct LVec;
+template <> struct LVec<double> {
+  typedef double v __attribute__((ext_vector_type(2), aligned(8)));
+  static constexpr int N = 2;
+};
+template <> struct LVec<float> {
+  typedef float v __attribute__((ext_vector_type(4), aligned(4)));
+  static constexpr int N = 4;
+};
+
+// A barrier that waits for LDS only: __syncthreads() also waits for the
+// published values to be in memory.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Sum of m[e] times the x of lane e of the lane's 16.
+template <class T>
+__device__ __forceinline__ T dot16(const T (&m)[16], T x) {
+  T p0 = T(0), p1 = T(0);
+  fmac_from<0>(p0, x, m[0]);   fmac_from<1>(p1, x, m[1]);
+  fmac_from<2>(p0, x, m[2]);   fmac_from<3>(p1, x, m[3]);
+  fmac_from<4>(p0, x, m[4]);   fmac_from<5>(p1, x, m[5]);
+  fmac_from<6>(p0, x, m[6]);   fmac_from<7>(p1, x, m[7]);
+  fmac_from<8>(p0, x, m[8]);   fmac_from<9>(p1, x, m[9]);
+  fmac_from<10>(p0, x, m[10]); fmac_from<11>(p1, x, m[11]);
+  fmac_from<12>(p0, x, m[12]); fmac_from<13>(p1, x, m[13]);
+  fmac_from<14>(p0, x, m[14]); fmac_from<15>(p1, x, m[15]);
+  return p0 + p1;
+}
+
+// Steps K .. 15 of the substitution in one 16 x 16 block.
+template <class T, Diag D, int K>
+__device__ __forceinline__ void diag_steps(T& x, T r, const T (*c)[17], int sub) {
+  if constexpr (K < 16) {
+    fmac_from<K>(x, by_diag<T, D>(x, r, r), c[K][sub]);
+    diag_steps<T, D, K + 1>(x, r, c, sub);
+  } else {
+    x = by_diag<T, D>(x, r, r);
+  }
+}
+
+// Sum over the 16 lanes of a row, in every lane.
+template <int ROR>
+__device__ __forceinline__ double ror16(double v) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, 0x120 + ROR, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), 0x120 + ROR, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+template <int ROR>
+__device__ __forceinline__ float ror16(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + ROR, 0xf, 0xf, true));
+}
+template <class T>
+__device__ __forceinline__ T sum16(T v) {
+  v += ror16<8>(v);
+  v += ror16<4>(v);
+  v += ror16<2>(v);
+  return v + ror16<1>(v);
+}
+
+template <class T>
+struct LineLds {
+  TriBlock<T> tri[2];
+  T inv[2][64][66];
+  T tmp[6][16][17];
+  T rec[RB];
+  T part[8][RB];  // the parts of a row's sum
+  T y[RB];
+  T x[64];        // the half solved first
+  int t, failed;
+};
+
+// The inverses of both triangles into S.inv, which holds zeros.  V in the order
+// of the substitution, by 16 x 16 blocks: V(i, i) by substitution, 16 lanes a
+// column; V(i, j) = V(i, i) sum over k = j .. i-1 of -M(i, k) V(k, j), the blocks
+// of equal i - j at once, a wave each.
+template <class T, bool LOWERM, bool UNIT>
+__device__ __forceinline__ void invert_triangles(LineLds<T>& S, int tid) {
+  typedef Mfma<T> MM;
+  const int lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto at = [](int i) { return LOWERM ? i : 63 - i; };
+#pragma unroll 1
+  for (int blk = 0; blk < 2; ++blk) {
+    const int m = wave >> 2, j = tid / 16 & 15;  // block m, column j
+    T x = li == j ? T(1) : T(0);
+    const T r = UNIT ? T(1) : S.rec[64 * blk + at(16 * m + li)];
+    diag_steps<T, UNIT ? DIAG_UNIT : DIAG_MULTIPLY, 0>(x, r, S.tri[blk].c[m * (m + 1) / 2 + m], li);
+    S.inv[blk][at(16 * m + li)][at(16 * m + j)] = x;
+  }
+#pragma unroll 1
+  for (int d = 1; d < 4; ++d) {
+    __syncthreads();
+    const int cnt = 4 - d;
+    if (wave < 2 * cnt) {
+      const int blk = wave >= cnt, j = wave - blk * cnt, i = j + d;
+      typename MM::acc_t acc = {T(0), T(0), T(0), T(0)};
+#pragma unroll 1
+      for (int k = j; k < i; ++k)
+#pragma unroll
+        for (int s = 0; s < 16; s += 4)
+          acc = MM::op(S.tri[blk].c[i * (i + 1) / 2 + k][s + lk][li], S.inv[blk][at(16 * k + s + lk)][at(16 * j + li)], acc);
+      T(*const tmp)[17] = S.tmp[wave];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tmp[MM::row(lk, r)][li] = acc[r];
+      wave_sync();
+      acc = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+      for (int s = 0; s < 16; s += 4) acc = MM::op(S.inv[blk][at(16 * i + li)][at(16 * i + s + lk)], tmp[s + lk][li], acc);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S.inv[blk][at(16 * i + MM::row(lk, r))][at(16 * j + li)] = acc[r];
+    }
+  }
+  __syncthreads();
+}
+
+template <class T, bool LOWERM, bool UNIT, bool TRANS>
+__global__ __launch_bounds__(1024) void tri_line_kernel(int n, const T* __restrict__ A, long lda,
+                                                        const T* __restrict__ Xin, T* __restrict__ X, unsigned* ticket,
+                                                        int* err) {
+  __shared__ LineLds<T> S;
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nblk = (n + RB - 1) / RB;
+  if (tid == 0) S.failed = 0;
+  if (tid == 0) S.t = (int)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const int t = __builtin_amdgcn_readfirstlane(S.t);
+  if (t >= nblk) return;
+  auto block_of = [&](int k) { return LOWERM ? k : nblk - 1 - k; };
+  const int r0 = RB * block_of(t);
+  auto M = [&](int i, int c) { return TRANS ? A[c + (long)i * lda] : A[i + (long)c * lda]; };
+
+  T b, mt[4];
+  // the diagonal triangles, in the order of the substitution, and the tile that
+  // takes the half solved first to the other (every load unconditional, at a
+  // clamped place, so that they are in flight together)
+  constexpr int F = LOWERM ? 0 : 1, L = 1 - F;
+  const int pr = tid >> 4, ps = tid & 15;  // row pr of a half, columns 4 ps .. + 3
+  {
+    const int a = tid & 15, c = (tid & 255) >> 4;  // a: the index that is contiguous in memory
+    auto place = [&](int u, int& blk, int& sb, int& gi, int& gk) {
+      const int s2 = tid / 256 + 4 * u;
+      blk = s2 >= 10;
+      sb = s2 - 10 * blk;
+      const int mi = sb >= 6 ? 3 : sb >= 3 ? 2 : sb >= 1 ? 1 : 0, mk = sb - mi * (mi + 1) / 2;
+      const int i = 16 * mi + (TRANS ? c : a), k = 16 * mk + (TRANS ? a : c);
+      gi = r0 + 64 * blk + (LOWERM ? i : 63 - i);
+      gk = r0 + 64 * blk + (LOWERM ? k : 63 - k);
+    };
+    auto at = [&](int i, int k) { return M(min(i, n - 1), min(k, n - 1)); };
+    T v[5], mt0[4];
+#pragma unroll
+    for (int u = 0; u < 5; ++u) {
+      int blk, sb, gi, gk;
+      place(u, blk, sb, gi, gk);
+      v[u] = at(gi, gk);
+    }
+    const int li2 = r0 + 64 * L + pr, lc2 = r0 + 64 * F + 4 * ps;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) mt0[j] = at(li2, lc2 + j);
+    const int g = min(r0 + (tid & (RB - 1)), n - 1);
+    const T b0 = Xin[g], d0 = UNIT ? T(1) : A[g + (long)g * lda];
+#pragma unroll
+    for (int u = 0; u < 5; ++u) {
+      int blk, sb, gi, gk;
+      place(u, blk, sb, gi, gk);
+      const bool in = (LOWERM ? gi > gk : gi < gk) && max(gi, gk) < n;
+      S.tri[blk].c[sb][TRANS ? a : c][TRANS ? c : a] = in ? -v[u] : T(0);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      mt[j] = li2 < n && lc2 + j < n ? mt0[j] : T(0);
+      asm volatile("" : "+v"(mt[j]));  // (here, not on the chain)
+    }
+    const bool in = r0 + (tid & (RB - 1)) < n;
+    b = in ? b0 : T(0);
+    if (tid < RB) S.rec[tid] = !UNIT && in ? T(1) / d0 : T(1);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) S.inv[u / 4][(tid >> 6) + 16 * (u & 3)][lane] = T(0);
+  }
+  __syncthreads();
+  invert_triangles<T, LOWERM, UNIT>(S, tid);
+  T inv[2][4];
+#pragma unroll
+  for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      inv[blk][j] = S.inv[blk][pr][4 * ps + j];
+      asm volatile("" : "+v"(inv[blk][j]));  // (kept: not read again on the chain)
+    }
+
+  // the tiles: wave w has, transposed, rows 16 (w / 2) .. and columns 64 (w % 2)
+  // .. (lane (li, lk): row li, columns 16 c + 4 lk + 0..3); otherwise rows 64 (w %
+  // 2) .. and columns 16 (w / 2) .. (a row a lane)
+  const int wr = TRANS ? 16 * (wave >> 1) : 64 * (wave & 1), wc = TRANS ? 64 * (wave & 1) : 16 * (wave >> 1);
+  const int row = min(r0 + wr + (TRANS ? li : lane), n - 1);
+  auto load = [&](T(&m)[16], int k) {
+    const int c0 = RB * block_of(k) + wc;
+    if (TRANS) {
+      typedef LVec<T> V;
+      const T* p = A + (long)row * lda;
+      if (c0 + 64 <= n) {
+        p += c0 + 4 * lk;
+#pragma unroll
+        for (int e = 0; e < 16; e += V::N) {
+          const typename V::v v = *reinterpret_cast<const typename V::v*>(p + 16 * (e / 4) + (e & 3));
+#pragma unroll
+          for (int q = 0; q < V::N; ++q) m[e + q] = v[q];
+        }
+      } else {
+        T v[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = p[min(c0 + 4 * lk + 16 * (e / 4) + (e & 3), n - 1)];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) m[e] = c0 + 4 * lk + 16 * (e / 4) + (e & 3) < n ? v[e] : T(0);
+      }
+    } else {
+      T v[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) v[e] = (A + (long)min(c0 + e, n - 1) * lda)[(unsigned)row];
+      if (c0 + 16 > n) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = c0 + e < n ? v[e] : T(0);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) m[e] = v[e];
+    }
+  };
+  bool failed = false;
+  T acc = T(0);
+  auto step = [&](const T(&m)[16], int k) {
+    // (value e of a lane's 16 is multiplied by the x that lane e of its row of 16 lanes holds)
+    const int c = RB * block_of(k) + wc + (TRANS ? 16 * (li >> 2) + 4 * lk + (li & 3) : li);
+    const T* const px = X + min(c, n - 1);
+    T x;
+    for (unsigned spins = 0;;) {
+      x = ld_dev(px);
+      if (!__any(is_sent(x))) break;
+      if (t - k > 2) __builtin_amdgcn_s_sleep(8);  // (its turn is not near: fewer loads)
+      else __builtin_amdgcn_s_sleep(1);
+      ++spins;
+      if ((spins & 255u) == 0u && ld_dev(err) != 0) { failed = true; return; }
+      if (spins > SPIN_LIMIT) { st_dev(err, 1); failed = true; return; }
+    }
+    x = c < n ? x : T(0);
+    acc += dot16(m, x);
+  };
+  T m0[16], m1[16];
+  if (t > 0) load(m0, 0);
+  for (int k = 0; k < t && !failed; k += 2) {
+    if (k + 1 < t) load(m1, k + 1);
+    step(m0, k);
+    if (k + 1 < t && !failed) {
+      if (k + 2 < t) load(m0, k + 2);
+      step(m1, k + 1);
+    }
+  }
+  if (failed && lane == 0) S.failed = 1;
+  S.part[TRANS ? 4 * (wave & 1) + lk : wave >> 1][wr + (TRANS ? li : lane)] = acc;
+  lds_barrier();
+  if (S.failed) return;
+  if (tid < RB) {
+    const T s0 = S.part[0][tid] + S.part[1][tid], s1 = S.part[2][tid] + S.part[3][tid];
+    const T s2 = S.part[4][tid] + S.part[5][tid], s3 = S.part[6][tid] + S.part[7][tid];
+    S.y[tid] = b - ((s0 + s1) + (s2 + s3));
+  }
+  lds_barrier();
+  // row pr of a 64 x 64 matrix times v
+  auto product = [&](const T(&a)[4], const T* v) {
+    const T p0 = fma(a[2], v[4 * ps + 2], a[0] * v[4 * ps]), p1 = fma(a[3], v[4 * ps + 3], a[1] * v[4 * ps + 1]);
+    return sum16(p0 + p1);
+  };
+  const T xf = product(inv[F], S.y + 64 * F);
+  if (ps == 0) S.x[pr] = xf;
+  lds_barrier();
+  if (ps == 0 && r0 + 64 * F + pr < n) st_dev(X + r0 + 64 * F + pr, canon(xf));
+  const T d = product(mt, S.x);
+  if (ps == 0) S.y[64 * L + pr] -= d;
+  lds_barrier();
+  const T xl = product(inv[L], S.y + 64 * L);
+  if (ps == 0 && r0 + 64 * L + pr < n) st_dev(X + r0 + 64 * L + pr, canon(xl));
+}
+
+}  // namespace
+
+// which: 0 = L (unit lower), 1 = U (upper), 2 = U^T, 3 = L^T.  X is filled with
+// the sentinel of getrs.hip and *ticket is 0.
+template <class T>
+void launch_tri_line(int which, int n, const T* A, long lda, const T* Xin, T* X, unsigned* ticket, int* err,
+                     hipStream_t s) {
+  const int nblk = (n + RB - 1) / RB;
+  switch (which) {
+    case 0: tri_line_kernel<T, true, true, false><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, X, ticket, err); break;
+    case 1: tri_line_kernel<T, false, false, false><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, X, ticket, err); break;
+    case 2: tri_line_kernel<T, true, false, true><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, X, ticket, err); break;
+    case 3: tri_line_kernel<T, false, true, true><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, X, ticket, err); break;
+  }
+}
+template void launch_tri_line<double>(int, int, const double*, long, const double*, double*, unsigned*, int*,
+                                      hipStream_t);
+template void launch_tri_line<float>(int, int, const float*, long, const float*, float*, unsigned*, int*, hipStream_t);
+
+}  // namespace la

@@ -1,0 +1,50 @@
+"""One right-hand side through DGETRS (SRC/dgetrs.f:181-218): the sweep by blocks of
+128 rows, at the edges of its blocks, halves and 16-row parts, against the
+oracle's DGETRS on the same factors and against the sweep that takes several
+right-hand sides.
+
+Tolerance: the matrices are random rows plus 4 sqrt(n) on the diagonal, their
+rows shuffled, so that |L||U| stays a small multiple of |A| and the condition
+number a small constant; every solution is then within a small multiple of
+n eps of the exact one (Higham, Accuracy and Stability, thm 9.4), taken as
+64 n eps.
+"""
+import numpy as np
+import pytest
+import torch
+
+import lapack_amd as la
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 300, 385, 900])
+def test_one_right_hand_side(dev, n, dtype):
+    dbl = dtype == np.float64
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((n, n)) + 4.0 * np.sqrt(n) * np.eye(n)
+    a = np.asfortranarray(a[rng.permutation(n)].astype(dtype))
+    lu, p = (oracle.dgetrf if dbl else oracle.sgetrf)(a)[:2]
+    b = rng.standard_normal((n, 3)).astype(dtype)
+    lda, ldb = n + 3, n + 5
+    buf = np.full((n, lda), np.nan, dtype=dtype)  # what lies between n and lda is not read
+    buf[:, :n] = lu.T
+    d_a, d_p = torch.from_numpy(buf).cuda(), torch.from_numpy(np.asarray(p, dtype=np.int32)).cuda()
+    tol = 64 * n * (2.0 ** -53 if dbl else 2.0 ** -24)
+    for trans in "NT":
+        ref = (oracle.dgetrs if dbl else oracle.sgetrs)(lu, p, np.asfortranarray(b), trans)[0]
+        got = []
+        for cols in ([0], [1], [0, 1, 2]):
+            host = np.full((len(cols), ldb), 55.0, dtype=dtype)
+            host[:, :n] = b[:, cols].T
+            d_b = torch.from_numpy(host).cuda()
+            rc = (la.dgetrs_async if dbl else la.sgetrs_async)(trans, n, len(cols), d_a, lda, d_p, d_b, ldb)
+            torch.cuda.synchronize()
+            assert rc == 0 and la.device_status() == 0
+            out = d_b.cpu().numpy()
+            assert (out[:, n:] == 55.0).all()
+            got.append(out[:, :n])
+        for x, r in ((got[0][0], ref[:, 0]), (got[1][0], ref[:, 1]), (got[0][0], got[2][0]), (got[1][0], got[2][1])):
+            assert np.abs(x - r).max() <= tol * np.abs(r).max(), (n, trans)
