@@ -931,26 +931,27 @@ void launch_gemm_t(char ta, char tb, int m, int n, int k, T alpha, const T* A, l
     gemm_kernel<T, true, true, false><<<grid, NT, 0, s>>>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tm, tn, chunk, nx);
 }
 
-// CUs per XCD a persistent update may hold (LAPACK_AMD_UPD_CUS, default 24
-// of 32: at n = 16384, 0.25-0.35 ms per factorization faster than 28; 22 and
-// 26 slower than 28, 16 by 5 ms, 32 by 9 ms).
+// CUs per XCD a persistent update may hold (LAPACK_AMD_UPD_CUS, default 28
+// of 32: DGETRF at n = 16384 / 12000 / 8192 takes 84.5 / 44.5 / 24.1 ms with 26 to
+// 28, 85.4 / 45.1 / 24.2 with 24, and 90.4 / 50.3 / 27.9 with 29: the panel's
+// short launches need four).
 static int update_cus_per_xcd() {
   static int v = -1;
   if (v < 0) {
     const char* e = std::getenv("LAPACK_AMD_UPD_CUS");
-    v = (e && *e) ? std::atoi(e) : 24;
+    v = (e && *e) ? std::atoi(e) : 28;
     if (v < 1) v = 1;
   }
   return v;
 }
 // The same for FP32 (LAPACK_AMD_UPD_CUS_S), whose update runs twice as fast:
-// DSGESV at n = 32768 took 401-404 ms with 20, 404-406 ms with 24, 404 ms
-// with 16 and 409 ms with 12.
+// SGETRF at n = 16384 / 12000 / 8192 takes 55.0 / 32.9 / 20.5 ms with 24, 54.8 / 33.1 /
+// 20.5 with 20 and 55.3 / 33.2 / 20.7 with 28.
 static int update_cus_per_xcd_s() {
   static int v = -1;
   if (v < 0) {
     const char* e = std::getenv("LAPACK_AMD_UPD_CUS_S");
-    v = (e && *e) ? std::atoi(e) : 20;
+    v = (e && *e) ? std::atoi(e) : 24;
     if (v < 1) v = 1;
   }
   return v;
@@ -958,13 +959,14 @@ static int update_cus_per_xcd_s() {
 
 // An update beside the panel below this many flops runs persistent on
 // update_cus_per_xcd() CUs per XCD (LAPACK_AMD_UPD_PERSIST_GF, in GFLOP;
-// default 60: at n = 16384, 30 is 0.5 ms per factorization slower, 90 and
-// 140 are 5 and 13 ms slower).
+// default 40, with the panel's workgroups on an XCD of their own: DGETRF at
+// n = 16384 / 12000 takes 84.6 / 44.6 ms with 30 and 40, 85.4 / 45.1 with 60,
+// 86.4 / 46.2 with 0; SGETRF 55.0 / 32.9 with 40, 56.4 / 33.3 with 90).
 static double update_persist_flops() {
   static double v = -1;
   if (v < 0) {
     const char* e = std::getenv("LAPACK_AMD_UPD_PERSIST_GF");
-    v = 1e9 * ((e && *e) ? std::atof(e) : 60.0);
+    v = 1e9 * ((e && *e) ? std::atof(e) : 40.0);
     if (v < 0) v = 0;
   }
   return v;
