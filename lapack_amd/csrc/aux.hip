@@ -486,8 +486,25 @@ __global__ __launch_bounds__(256) void copy_kernel(int rows, int cols, const T* 
     dst[i + j * ldd] = src[i + j * lds];
   }
 }
-__global__ void fold_err_kernel(const int* __restrict__ err, int* __restrict__ info, int* __restrict__ sticky) {
-  if (threadIdx.x == 0 && *err) {
+// Start of a factorization: the exchange buffer's words zero, the wait-error word
+// (fail: the test hook) and INFO.
+__global__ __launch_bounds__(256) void lu_init_kernel(unsigned* __restrict__ words, size_t n, int* __restrict__ err,
+                                                      int fail, int* __restrict__ info) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) words[i] = 0u;
+  if (i == 0) {
+    *err = fail;
+    *info = 0;
+  }
+}
+// The wait-error word of a solve: set by the test hook, and where *gate (the
+// factorization's INFO; may be null) calls the solve off.
+__global__ void solve_err_kernel(int* __restrict__ err, int fail, const int* __restrict__ gate) {
+  if (threadIdx.x == 0) *err = fail || (gate && *gate != 0);
+}
+__global__ void fold_err_kernel(const int* __restrict__ err, int* __restrict__ info, int* __restrict__ sticky,
+                                const int* __restrict__ gate) {
+  if (threadIdx.x == 0 && *err && !(gate && *gate != 0)) {
     if (info) *info = LA_ERR_SYNC;
     if (sticky) atomicOr(sticky, 1);
   }
@@ -649,8 +666,14 @@ void launch_fill_u32(unsigned* p, size_t n, unsigned v, hipStream_t s) {
 void launch_fill_random(double* x, size_t n, unsigned long long seed, hipStream_t s) {
   if (n) fill_random_kernel<<<grid_for((long)std::min<size_t>(n, (size_t)1 << 40)), 256, 0, s>>>(x, n, seed);
 }
-void launch_fold_err(const int* err, int* info, int* sticky, hipStream_t s) {
-  fold_err_kernel<<<1, 64, 0, s>>>(err, info, sticky);
+void launch_lu_init(unsigned* words, size_t n, int* err, int fail, int* info, hipStream_t s) {
+  lu_init_kernel<<<(unsigned)((std::max<size_t>(n, 1) + 255) / 256), 256, 0, s>>>(words, n, err, fail, info);
+}
+void launch_solve_err(int* err, int fail, const int* gate, hipStream_t s) {
+  solve_err_kernel<<<1, 64, 0, s>>>(err, fail, gate);
+}
+void launch_fold_err(const int* err, int* info, int* sticky, hipStream_t s, const int* gate) {
+  fold_err_kernel<<<1, 64, 0, s>>>(err, info, sticky, gate);
 }
 void launch_fill_i32(int* p, size_t n, int v, hipStream_t s) {
   if (n) fill_kernel<int><<<grid_for((long)n), 256, 0, s>>>(p, n, v);

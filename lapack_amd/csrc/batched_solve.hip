@@ -165,40 +165,6 @@ __device__ __forceinline__ void sweep(const T* A, long lda, int n, T* X, int ldx
   }
 }
 
-// Interchanges of X by one wave: in order (SRC/dgetrs.f:187), or in reverse
-// order (:217).  Pivots outside the matrix move nothing.
-template <class T, bool REVERSE>
-__device__ __forceinline__ void interchange(const int* ipiv, int n, T* X, int ldx, int nr, int lane) {
-  const int nblk = (n + 63) / 64;
-  for (int ib = 0; ib < nblk; ++ib) {
-    const int k0 = 64 * (REVERSE ? nblk - 1 - ib : ib);
-    int p = k0 + lane;
-    if (p < n) {
-      const int v = ipiv[p] - 1;
-      if (v >= 0 && v < n) p = v;
-    }
-    int from_k = k0 + lane, from_p = p;
-    const int cnt = min(64, n - k0);
-#pragma unroll 4
-    for (int j = 0; j < cnt; ++j) {
-      const int jj = REVERSE ? j : cnt - 1 - j;
-      const int k = k0 + jj, pk = __builtin_amdgcn_readlane(p, jj);
-      from_k = from_k == k ? pk : from_k == pk ? k : from_k;
-      from_p = from_p == k ? pk : from_p == pk ? k : from_p;
-    }
-    if (k0 + lane < n) {
-      for (int q = 0; q < nr; ++q) {
-        T* x = X + q * ldx;
-        const T a = x[from_k], b = x[from_p];
-        wave_sync();
-        x[k0 + lane] = a;
-        x[p] = b;
-      }
-    }
-    wave_sync();
-  }
-}
-
 // The reference's order with its zero tests, for matrices whose result is not
 // finite.  X holds B with its rows interchanged (N) or B (T).
 template <class T, bool TRANS, int NT, int NR>

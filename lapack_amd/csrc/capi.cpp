@@ -29,7 +29,7 @@ template <class T>
 int getrs_device(char trans, int n, int nrhs, const T* A, long lda, const int* ipiv, T* B, long ldb, hipStream_t s);
 template <class T>
 int getrs_device_ex(char trans, int n, int nrhs, const T* A, long lda, const int* ipiv, T* B, long ldb, hipStream_t s,
-                    int* waitflag);
+                    int* waitflag, const int* gate);
 int with_safe_forms(const std::function<int()>& f);
 void fail_waits(int count);
 int device_status(int clear);
@@ -261,7 +261,7 @@ int getrs_sync(char trans, int n, int nrhs, const T* a, int lda, const int* ipiv
   int flag = 0;
   auto solve = [&]() -> int {
     launch_fill_i32(dflag, 1, 0, call.s);
-    int r = getrs_device_ex<T>(trans, n, nrhs, A.dev, A.ld, P.dev, B.dev, B.ld, call.s, dflag);
+    int r = getrs_device_ex<T>(trans, n, nrhs, A.dev, A.ld, P.dev, B.dev, B.ld, call.s, dflag, nullptr);
     if (r) return r;
     if ((r = to_host(B, call.s))) return r;
     CK(hipMemcpyAsync(&flag, dflag, sizeof(int), hipMemcpyDeviceToHost, call.s));
@@ -303,20 +303,36 @@ int gesv_sync(int n, int nrhs, double* a, int lda, int* ipiv, double* b, int ldb
     CK(hipStreamSynchronize(call.s));
     return 0;
   };
-  auto solve = [&]() -> int {
+  auto enqueue_solve = [&](const int* gate) -> int {
     launch_fill_i32(dinfo + 1, 1, 0, call.s);
-    int r = getrs_device_ex<double>('N', n, nrhs, A.dev, A.ld, P.dev, B.dev, B.ld, call.s, dinfo + 1);
+    return getrs_device_ex<double>('N', n, nrhs, A.dev, A.ld, P.dev, B.dev, B.ld, call.s, dinfo + 1, gate);
+  };
+  auto solve = [&]() -> int {
+    int r = enqueue_solve(nullptr);
     if (r) return r;
     CK(hipMemcpyAsync(&flag, dinfo + 1, sizeof(int), hipMemcpyDeviceToHost, call.s));
     CK(hipStreamSynchronize(call.s));
     return 0;
   };
-  if ((rc = factor())) return rc;
+  // The solve follows the factorization without a look at INFO in between: it
+  // leaves B alone where INFO is not 0.
+  if ((rc = getrf_device<double>(n, n, A.dev, A.ld, P.dev, dinfo, call.s))) return rc;
+  const int rs = nrhs > 0 ? enqueue_solve(dinfo) : 0;
+  int both[2] = {0, 0};
+  CK(hipMemcpyAsync(both, dinfo, sizeof(int) * (nrhs > 0 ? 2 : 1), hipMemcpyDeviceToHost, call.s));
+  CK(hipStreamSynchronize(call.s));
+  info = both[0];
+  flag = both[1];
+  const bool again = info == LA_ERR_SYNC;
   // a bounded wait gave up: A was left as passed; factor it again without waits
-  if (info == LA_ERR_SYNC && (rc = with_safe_forms(factor))) return rc;
+  if (again && (rc = with_safe_forms(factor))) return rc;
   // DGESV solves only when the factorization is nonsingular (SRC/dgesv.f:170-175).
   if (info == 0 && nrhs > 0) {
-    if ((rc = solve())) return rc;
+    if (again) {
+      if ((rc = solve())) return rc;
+    } else if (rs) {
+      return rs;
+    }
     if (flag && (rc = with_safe_forms(solve))) return rc;
     if (flag) info = LA_ERR_SYNC;
   }

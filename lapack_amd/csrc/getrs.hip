@@ -457,7 +457,8 @@ void launch_chain(int n, int nrhs, const T* A, long lda, const T* Xin, long ldxi
 
 }  // namespace
 
-size_t tri_chain_ctl_words(int nrhs) { return (size_t)std::max(1, (nrhs + TQ - 1) / TQ); }
+// (two at least: one right-hand side has a ticket for each of its sweeps)
+size_t tri_chain_ctl_words(int nrhs) { return (size_t)std::max(2, (nrhs + TQ - 1) / TQ); }
 
 // which: 0 = L (unit lower), 1 = U (upper), 2 = U^T, 3 = L^T.
 template <class T>

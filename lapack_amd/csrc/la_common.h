@@ -118,7 +118,11 @@ void launch_fill_i32(int* p, size_t n, int v, hipStream_t s);
 void launch_fill_random(double* x, size_t n, unsigned long long seed, hipStream_t s);
 // When a bounded wait gave up (*err != 0): *info <- LA_ERR_SYNC and bit 0 of
 // *sticky set (either pointer may be null).
-void launch_fold_err(const int* err, int* info, int* sticky, hipStream_t s);
+void launch_fold_err(const int* err, int* info, int* sticky, hipStream_t s, const int* gate = nullptr);
+// words zero, *err = fail, *info = 0
+void launch_lu_init(unsigned* words, size_t n, int* err, int fail, int* info, hipStream_t s);
+// *err = fail, or 1 where *gate (may be null) is not 0
+void launch_solve_err(int* err, int fail, const int* gate, hipStream_t s);
 
 // Panel (leaf) factorization on the transposed workspace: see panel.hip.
 // xchg (panel_xchg_bytes() bytes) must be zero at the start of a
@@ -211,7 +215,13 @@ template <class T>
 int launch_getrf_batched_leaf(const BatchedLeafPlan& p, const int* nv, T* const* av, const int* ldav, int* const* ipv,
                               int* infov, const int* order, unsigned* counters, hipStream_t s);
 
-// One right-hand side (tri_line.hip).
+// DGETRS of one right-hand side (tri_line.hip): b is replaced unless *gate (may be
+// null) is not 0 or a wait gives up; X, Y: n values; tickets: two words.
+template <class T>
+void launch_getrs_line(bool notran, int n, const T* A, long lda, const int* ipiv, T* b, T* X, T* Y, unsigned* tickets,
+                       int* err, int* perm, int* gpairs, bool fail, const int* gate, int* waitflag, int* sticky,
+                       hipStream_t s);
+// One of its sweeps.
 template <class T>
 void launch_tri_line(int which, int n, const T* A, long lda, const T* Xin, T* X, unsigned* ticket, int* err,
                      hipStream_t s);

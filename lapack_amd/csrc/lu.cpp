@@ -536,9 +536,8 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
   // the panel's flag-in-data exchange needs a zeroed buffer per factorization;
   // the flag base starts over only long before it could wrap
   if (c->leaf_tag > 0xF0000000u) c->leaf_tag = 0;
-  launch_fill_u32(reinterpret_cast<unsigned*>(xchg), panel_xchg_bytes(0) / sizeof(unsigned), 0u, s);
-  launch_fill_i32(err, 1, fail > 0 ? 1 : 0, s);
-  launch_fill_i32(info, 1, 0, s);
+  launch_lu_init(reinterpret_cast<unsigned*>(xchg), panel_xchg_bytes(0) / sizeof(unsigned), err, fail > 0 ? 1 : 0, info,
+                 s);
   mark(pa, fla, LA_PHASE_TRANSPOSE, 0);
   K<T>::transpose(m, n, A, lda, Tm, ldt, s);  // T(c, r) = A(r, c)
   endm(pa, fla);
@@ -698,10 +697,12 @@ size_t getrs_ws_bytes(int n, int nrhs, int nbs) {
 // permutation, then one tri_chain launch per triangular sweep (getrs.hip).
 // When a wait gives up, B is left as passed and the failure is folded into
 // *waitflag and *sticky (device ints; either may be null).  fail: start with
-// the wait-error word set (the test hook).  Enqueued on s; allocates nothing.
+// the wait-error word set (the test hook).  gate (a device int, or null): where
+// it is not 0 when the solve starts, B is left as passed and nothing is
+// reported.  Enqueued on s; allocates nothing.
 template <class T>
 void getrs_chain(char trans, int n, int nrhs, const T* A, long lda, const int* ipiv, T* B, long ldb, char* ws,
-                 bool fail, int* waitflag, int* sticky, hipStream_t s) {
+                 bool fail, int* waitflag, int* sticky, hipStream_t s, const int* gate) {
   const bool notran = (trans == 'N' || trans == 'n');
   Carve cv;
   int* perm = reinterpret_cast<int*>(ws + cv.take<int>((size_t)n));
@@ -711,7 +712,11 @@ void getrs_chain(char trans, int n, int nrhs, const T* A, long lda, const int* i
   int* cerr = reinterpret_cast<int*>(ws + cv.take<int>(1));
   int* gpairs = reinterpret_cast<int*>(ws + cv.take<int>(perm_pairs_ints(0, n)));
   const long ldx = n;
-  launch_fill_i32(cerr, 1, fail ? 1 : 0, s);
+  if (nrhs == 1) {
+    launch_getrs_line<T>(notran, n, A, lda, ipiv, B, X, Y, ctl, cerr, perm, gpairs, fail, gate, waitflag, sticky, s);
+    return;
+  }
+  launch_solve_err(cerr, fail ? 1 : 0, gate, s);
   if (notran) {
     launch_swaps_to_perm(n, 0, n, ipiv, 1, perm, s, gpairs);
     K<T>::gather(n, nrhs, perm, B, ldb, X, ldx, s);                         // X = P*B (dgetrs.f:187)
@@ -725,7 +730,7 @@ void getrs_chain(char trans, int n, int nrhs, const T* A, long lda, const int* i
     launch_swaps_to_perm(n, 0, n, ipiv, -1, perm, s, gpairs);                // dgetrs.f:217
     K<T>::gather(n, nrhs, perm, X, ldx, B, ldb, s, cerr);
   }
-  launch_fold_err(cerr, waitflag, sticky, s);
+  launch_fold_err(cerr, waitflag, sticky, s, gate);
 }
 
 // Solve op(A) X = B with the LU of getrf (SRC/dgetrs.f:181-218).  Device
@@ -740,7 +745,7 @@ void getrs_chain(char trans, int n, int nrhs, const T* A, long lda, const int* i
 //     blocks of L and U inverted once, every block step two MFMA GEMMs.
 template <class T>
 int getrs_device_ex(char trans, int n, int nrhs, const T* A, long lda, const int* ipiv, T* B, long ldb,
-                    hipStream_t s, int* waitflag) {
+                    hipStream_t s, int* waitflag, const int* gate) {
   DevCtx* c = get_ctx();
   if (!c) return LA_ERR_NODEVICE;
   std::lock_guard<std::mutex> g(c->mu);
@@ -763,7 +768,7 @@ int getrs_device_ex(char trans, int n, int nrhs, const T* A, long lda, const int
     int fail = g_fail_waits.load();
     while (fail > 0 && !g_fail_waits.compare_exchange_weak(fail, fail - 1)) {
     }
-    getrs_chain<T>(trans, n, nrhs, A, lda, ipiv, B, ldb, ws, fail > 0, waitflag, c->status, s);
+    getrs_chain<T>(trans, n, nrhs, A, lda, ipiv, B, ldb, ws, fail > 0, waitflag, c->status, s, gate);
     if (pt.mark(-1)) fl.push_back(0);
     rc = ws_release(c, s);
     phase_collect(pt, fl);
@@ -828,7 +833,7 @@ int getrs_device_ex(char trans, int n, int nrhs, const T* A, long lda, const int
 template <class T>
 int getrs_device(char trans, int n, int nrhs, const T* A, long lda, const int* ipiv, T* B, long ldb,
                  hipStream_t s) {
-  return getrs_device_ex<T>(trans, n, nrhs, A, lda, ipiv, B, ldb, s, nullptr);
+  return getrs_device_ex<T>(trans, n, nrhs, A, lda, ipiv, B, ldb, s, nullptr, nullptr);
 }
 
 // DLASWP on a column-major device matrix (SRC/dlaswp.f:112-189).  nrows is
@@ -883,12 +888,12 @@ template int getrf_device<float>(int, int, float*, long, int*, int*, hipStream_t
 template int getrs_device<double>(char, int, int, const double*, long, const int*, double*, long, hipStream_t);
 template int getrs_device<float>(char, int, int, const float*, long, const int*, float*, long, hipStream_t);
 template int getrs_device_ex<double>(char, int, int, const double*, long, const int*, double*, long, hipStream_t,
-                                     int*);
+                                     int*, const int*);
 template int getrs_device_ex<float>(char, int, int, const float*, long, const int*, float*, long, hipStream_t,
-                                    int*);
+                                    int*, const int*);
 template size_t getrs_chain_ws_bytes<double>(int, int);
 template void getrs_chain<double>(char, int, int, const double*, long, const int*, double*, long, char*, bool, int*,
-                                  int*, hipStream_t);
+                                  int*, hipStream_t, const int*);
 template int laswp_device<double>(int, double*, long, int, int, int, const int*, int, hipStream_t);
 template int laswp_device<float>(int, float*, long, int, int, int, const int*, int, hipStream_t);
 

@@ -29,7 +29,7 @@ template <class T>
 size_t getrs_chain_ws_bytes(int n, int nrhs);
 template <class T>
 void getrs_chain(char trans, int n, int nrhs, const T* A, long lda, const int* ipiv, T* B, long ldb, char* ws,
-                 bool fail, int* waitflag, int* sticky, hipStream_t s);
+                 bool fail, int* waitflag, int* sticky, hipStream_t s, const int* gate);
 }  // namespace la
 
 namespace {
@@ -93,7 +93,7 @@ int lapack_amd_dgetrs_noalloc_async(char trans, int n, int nrhs, const double* d
   if (!ws) return rc;
   la::launch_fill_i32(d_info, 1, 0, s);
   if (n > 0 && nrhs > 0)
-    la::getrs_chain<double>(trans, n, nrhs, d_a, lda, d_ipiv, d_b, ldb, ws, false, d_info, nullptr, s);
+    la::getrs_chain<double>(trans, n, nrhs, d_a, lda, d_ipiv, d_b, ldb, ws, false, d_info, nullptr, s, nullptr);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : LA_ERR_HIP;
 }

@@ -22,7 +22,8 @@
 // tile of 128 KB at what one CU gets from memory, 30 to 50 GB/s; 1.4 of it the
 // way of x through memory.  64-row blocks of 4 waves with a round's x in LDS took
 // 2.5 to 6.4 us for half the rows.  n = 6001, one right-hand side, FP64, with
-// the permutation: 'N' 541 -> 396 us, 'T' 978 -> 490; n = 100 84 -> 66.
+// the permutation: 'N' 541 -> 379 us, 'T' 978 -> 468; n = 100 84 -> 43 (launches: one
+// that clears, one that permutes up to 512 rows, the sweeps and one that ends).
 // Every wait is bounded; one that gives up sets *err, and the others poll *err
 // and give up as well, so every workgroup runs to its end.
 #include "tri_block.h"
@@ -151,9 +152,8 @@ __device__ __forceinline__ void invert_triangles(LineLds<T>& S, int tid) {
 }
 
 template <class T, bool LOWERM, bool UNIT, bool TRANS>
-__global__ __launch_bounds__(1024) void tri_line_kernel(int n, const T* __restrict__ A, long lda,
-                                                        const T* __restrict__ Xin, T* __restrict__ X, unsigned* ticket,
-                                                        int* err) {
+__global__ __launch_bounds__(1024) void tri_line_kernel(int n, const T* __restrict__ A, long lda, T* Xin, bool refill,
+                                                        T* __restrict__ X, unsigned* ticket, int* err) {
   __shared__ LineLds<T> S;
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -216,6 +216,9 @@ __global__ __launch_bounds__(1024) void tri_line_kernel(int n, const T* __restri
     for (int u = 0; u < 8; ++u) S.inv[u / 4][(tid >> 6) + 16 * (u & 3)][lane] = T(0);
   }
   __syncthreads();
+  // (a block's right side is read by its own workgroup only: its place can wait
+  // for the values of the next sweep)
+  if (refill && tid < RB && r0 + tid < n) Xin[r0 + tid] = __builtin_bit_cast(T, Sent<T>::bits);
   invert_triangles<T, LOWERM, UNIT>(S, tid);
   T inv[2][4];
 #pragma unroll
@@ -318,23 +321,126 @@ __global__ __launch_bounds__(1024) void tri_line_kernel(int n, const T* __restri
   if (ps == 0 && r0 + 64 * L + pr < n) st_dev(X + r0 + 64 * L + pr, canon(xl));
 }
 
+// A wait gave up (not where the solve was called off by the factorization's INFO).
+__device__ __forceinline__ void report_wait(int* waitflag, int* sticky, const int* gate) {
+  if (gate && *gate != 0) return;
+  if (waitflag) *waitflag = LA_ERR_SYNC;
+  if (sticky) atomicOr(sticky, 1);
+}
+
+// Start of a solve: the wait-error word (set where the factorization has an INFO,
+// and by the test hook), the sweeps' tickets, the first sweep's sentinels and, for a
+// b that is not interchanged first, its right side.
+template <class T>
+__global__ __launch_bounds__(256) void line_init_kernel(int n, const T* __restrict__ b, T* X, T* Y, unsigned* tickets,
+                                                        int* err, int fail, const int* __restrict__ gate) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) Y[i] = __builtin_bit_cast(T, Sent<T>::bits);
+  if (b && i < n) X[i] = b[i];
+  if (i < 2) tickets[i] = 0u;
+  if (i == 0) *err = fail || (gate && *gate != 0);
+}
+
+// End of a solve: dst = src unless a wait gave up, which is reported instead.
+template <class T>
+__global__ __launch_bounds__(256) void line_end_kernel(int n, const T* __restrict__ src, T* __restrict__ dst,
+                                                       const int* __restrict__ err, int* waitflag, int* sticky,
+                                                       const int* __restrict__ gate) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const bool failed = *err != 0;
+  if (!failed && i < n) dst[i] = src[i];
+  if (failed && i == 0) report_wait(waitflag, sticky, gate);
+}
+
+// dst = src with its rows interchanged, for columns that fit in LDS: one
+// workgroup, the interchanges composed by its first wave (11 us at n = 512
+// where composing them for any n, with the gather, takes three launches and 23).
+// err: nothing is written where it is set, but it is reported.
+constexpr int PERM_NMAX = 512;
+template <class T, bool REVERSE>
+__global__ __launch_bounds__(256) void permute_small_kernel(int n, const int* __restrict__ ipiv,
+                                                            const T* __restrict__ src, T* __restrict__ dst,
+                                                            const int* __restrict__ err, int* waitflag, int* sticky,
+                                                            const int* __restrict__ gate) {
+  __shared__ T x[PERM_NMAX];
+  const int tid = threadIdx.x;
+  if (err && *err != 0) {
+    if (tid == 0) report_wait(waitflag, sticky, gate);
+    return;
+  }
+  for (int i = tid; i < n; i += 256) x[i] = src[i];
+  __syncthreads();
+  if (tid < 64) interchange<T, REVERSE>(ipiv, n, x, 0, 1, tid);
+  __syncthreads();
+  for (int i = tid; i < n; i += 256) dst[i] = x[i];
+}
+
+void gather(int n, const int* perm, const double* src, double* dst, hipStream_t s) {
+  launch_gather_rows_d(n, 1, perm, src, n, dst, n, s);
+}
+void gather(int n, const int* perm, const float* src, float* dst, hipStream_t s) {
+  launch_gather_rows_s(n, 1, perm, src, n, dst, n, s);
+}
+
+template <class T>
+void launch_line(int which, int n, const T* A, long lda, T* Xin, bool refill, T* X, unsigned* ticket, int* err,
+                 hipStream_t s) {
+  const int nblk = (n + RB - 1) / RB;
+  switch (which) {
+    case 0: tri_line_kernel<T, true, true, false><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, refill, X, ticket, err); break;
+    case 1: tri_line_kernel<T, false, false, false><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, refill, X, ticket, err); break;
+    case 2: tri_line_kernel<T, true, false, true><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, refill, X, ticket, err); break;
+    case 3: tri_line_kernel<T, false, true, true><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, refill, X, ticket, err); break;
+  }
+}
+
 }  // namespace
 
 // which: 0 = L (unit lower), 1 = U (upper), 2 = U^T, 3 = L^T.  X is filled with
-// the sentinel of getrs.hip and *ticket is 0.
+// the sentinel and *ticket is 0.
 template <class T>
 void launch_tri_line(int which, int n, const T* A, long lda, const T* Xin, T* X, unsigned* ticket, int* err,
                      hipStream_t s) {
-  const int nblk = (n + RB - 1) / RB;
-  switch (which) {
-    case 0: tri_line_kernel<T, true, true, false><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, X, ticket, err); break;
-    case 1: tri_line_kernel<T, false, false, false><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, X, ticket, err); break;
-    case 2: tri_line_kernel<T, true, false, true><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, X, ticket, err); break;
-    case 3: tri_line_kernel<T, false, true, true><<<nblk, 1024, 0, s>>>(n, A, lda, Xin, X, ticket, err); break;
-  }
+  launch_line<T>(which, n, A, lda, const_cast<T*>(Xin), false, X, ticket, err, s);
 }
 template void launch_tri_line<double>(int, int, const double*, long, const double*, double*, unsigned*, int*,
                                       hipStream_t);
 template void launch_tri_line<float>(int, int, const float*, long, const float*, float*, unsigned*, int*, hipStream_t);
+
+// DGETRS of one right-hand side b (SRC/dgetrs.f:181-218): X and Y n values,
+// tickets two words, perm and gpairs as launch_swaps_to_perm takes them.
+template <class T>
+void launch_getrs_line(bool notran, int n, const T* A, long lda, const int* ipiv, T* b, T* X, T* Y, unsigned* tickets,
+                       int* err, int* perm, int* gpairs, bool fail, const int* gate, int* waitflag, int* sticky,
+                       hipStream_t s) {
+  const int nb = (n + 255) / 256;
+  line_init_kernel<T><<<nb, 256, 0, s>>>(n, notran ? nullptr : b, X, Y, tickets, err, fail ? 1 : 0, gate);
+  const bool small = n <= PERM_NMAX;
+  if (notran) {
+    if (small) {
+      permute_small_kernel<T, false><<<1, 256, 0, s>>>(n, ipiv, b, X, nullptr, nullptr, nullptr, nullptr);
+    } else {
+      launch_swaps_to_perm(n, 0, n, ipiv, 1, perm, s, gpairs);
+      gather(n, perm, b, X, s);
+    }
+    launch_line<T>(0, n, A, lda, X, true, Y, tickets, err, s);
+    launch_line<T>(1, n, A, lda, Y, false, X, tickets + 1, err, s);
+    line_end_kernel<T><<<nb, 256, 0, s>>>(n, X, b, err, waitflag, sticky, gate);
+    return;
+  }
+  launch_line<T>(2, n, A, lda, X, true, Y, tickets, err, s);
+  launch_line<T>(3, n, A, lda, Y, false, X, tickets + 1, err, s);
+  if (small) {
+    permute_small_kernel<T, true><<<1, 256, 0, s>>>(n, ipiv, X, b, err, waitflag, sticky, gate);
+  } else {
+    launch_swaps_to_perm(n, 0, n, ipiv, -1, perm, s, gpairs);
+    gather(n, perm, X, Y, s);
+    line_end_kernel<T><<<nb, 256, 0, s>>>(n, Y, b, err, waitflag, sticky, gate);
+  }
+}
+template void launch_getrs_line<double>(bool, int, const double*, long, const int*, double*, double*, double*,
+                                        unsigned*, int*, int*, int*, bool, const int*, int*, int*, hipStream_t);
+template void launch_getrs_line<float>(bool, int, const float*, long, const int*, float*, float*, float*, unsigned*,
+                                       int*, int*, int*, bool, const int*, int*, int*, hipStream_t);
 
 }  // namespace la

@@ -20,7 +20,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 300, 385, 900])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 300, 385, 512, 513,
+                               900])
 def test_one_right_hand_side(dev, n, dtype):
     dbl = dtype == np.float64
     rng = np.random.default_rng(n)
@@ -48,3 +49,30 @@ def test_one_right_hand_side(dev, n, dtype):
             got.append(out[:, :n])
         for x, r in ((got[0][0], ref[:, 0]), (got[1][0], ref[:, 1]), (got[0][0], got[2][0]), (got[1][0], got[2][1])):
             assert np.abs(x - r).max() <= tol * np.abs(r).max(), (n, trans)
+
+
+@pytest.mark.parametrize("nrhs", [1, 3])
+@pytest.mark.parametrize("n", [40, 100, 512, 513, 700])
+def test_gesv_solves_only_the_nonsingular(dev, n, nrhs):
+    """DGESV enqueues the solve behind the factorization: where INFO is not 0 it
+    leaves B and the device's status alone (SRC/dgesv.f:170-175)."""
+    rng = np.random.default_rng(n + nrhs)
+    a = rng.standard_normal((n, n)) + 4.0 * np.sqrt(n) * np.eye(n)
+    a = a[rng.permutation(n)]
+    b = rng.standard_normal((n, nrhs))
+    for singular in (False, True):
+        m = a.copy()
+        if singular:
+            m[:, n // 2] = 0.0
+        d_a, d_b = torch.from_numpy(m.T.copy()).cuda(), torch.from_numpy(b.T.copy()).cuda()
+        d_p = torch.zeros(n, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        info = la.dgesv(n, nrhs, d_a, n, d_p, d_b, n)
+        x = d_b.cpu().numpy().T
+        assert la.device_status() == 0
+        if singular:
+            assert info == n // 2 + 1
+            np.testing.assert_array_equal(x, b)
+        else:
+            assert info == 0
+            assert oracle.dget02(np.asfortranarray(m), np.asfortranarray(x), np.asfortranarray(b)) < 30.0
