@@ -219,13 +219,52 @@ __device__ __forceinline__ bool recip_ok(T piv) {
 // 64 per launch).
 constexpr int LG = 8;                        // columns of a group
 constexpr int MSGS = 32;                     // words of a candidate's slot (padded)
-constexpr size_t MSG_PAR = (size_t)(GMAX + 1) * MSGS;  // candidates of one column + row k
+constexpr size_t MSG_PAR = 2880;             // candidates of one column + row k
 constexpr int ROWS_SLOTS = 2 * LG;           // rows an 8-column group's interchanges touch
 constexpr int NOSLOT = 31;                   // a row no interchange of the group has touched
 constexpr size_t LL_WORDS = 2 * MSG_PAR + (size_t)ROWS_SLOTS * 2 * WMAX;
 
 __device__ __forceinline__ u64 ll_word(unsigned payload, unsigned flag) {
   return ((u64)flag << 32) | (u64)payload;
+}
+
+// Up to 128 waves (16 workgroups of 8) exchange without a workgroup's own fold in
+// between: each publishes its candidate's key -- the value, with the row's lane
+// and slot beside a 20-bit flag in the upper word -- and then its values; every
+// wave polls all the keys, one (DIRECT = 1) or two candidates a lane, folds them
+// and reads the winner's values.  That leaves out the fold between two barriers
+// (about 1000 of 5450 cycles a column) and takes the reciprocal out of the chain;
+// a round of loads is what the polls take more as the waves grow (DGETRF at n =
+// 1024 / 4096 / 8192: 2.30 / 10.86 / 24.04 -> 2.18 / 10.04 / 23.04 ms, SGETRF 2.03 /
+// 9.58 / 20.52 -> 1.88 / 8.46 / 18.56).  A flag's top bit tells these upper words from the other ones (whose
+// flags stay below 2^31).
+constexpr int DIRECT_CANDS = 128;
+constexpr int DIRECT_ROWK = 2 * DIRECT_CANDS;     // row k's words
+constexpr int DIRECT_VALUES = DIRECT_ROWK + 32;   // the candidates' values
+constexpr unsigned DIRECT_NONE = 1u << 11;
+static_assert(DIRECT_VALUES + DIRECT_CANDS * (2 * (LG + 1) + 2) <= MSG_PAR && (GMAX + 1) * MSGS <= MSG_PAR,
+              "the candidates' buffer");
+__device__ __forceinline__ unsigned direct_flag(unsigned flag, unsigned meta) {
+  return (0x80000u | (flag & 0x7ffffu)) << 12 | meta;
+}
+// word w of a value (0: the lower half), a value of its words, and of the words
+// that lanes l (and l + 1) hold (uniform)
+__device__ __forceinline__ unsigned value_word(double x, int w) {
+  return (unsigned)((u64)__double_as_longlong(x) >> (32 * w));
+}
+__device__ __forceinline__ unsigned value_word(float x, int) { return __float_as_uint(x); }
+template <class T> __device__ __forceinline__ T value_of(unsigned top, unsigned low);
+template <> __device__ __forceinline__ double value_of<double>(unsigned top, unsigned low) {
+  return __longlong_as_double((long long)((u64)top << 32 | low));
+}
+template <> __device__ __forceinline__ float value_of<float>(unsigned top, unsigned) { return __uint_as_float(top); }
+template <class T> __device__ __forceinline__ T word_value(int words, int l);
+template <> __device__ __forceinline__ double word_value<double>(int words, int l) {
+  return value_of<double>((unsigned)__builtin_amdgcn_readlane(words, l + 1),
+                          (unsigned)__builtin_amdgcn_readlane(words, l));
+}
+template <> __device__ __forceinline__ float word_value<float>(int words, int l) {
+  return __uint_as_float((unsigned)__builtin_amdgcn_readlane(words, l));
 }
 
 // ---- register-resident leaf ------------------------------------------------------
@@ -246,6 +285,8 @@ __device__ __forceinline__ u64 ll_word(unsigned payload, unsigned flag) {
 //   C   every wave folds the candidates; the winner's values come out of the
 //       fold's registers as scalars (readlane);
 //   D   interchange, scaling, update of the group's remaining columns.
+// (With up to 16 workgroups every wave publishes its candidate instead, and
+// folds all of them: no barrier inside a group.)
 // Buffers alternate with the column parity, so no barrier ends a column.
 // After each group:
 //   E   the at most 16 rows that the group's interchanges touch go through
@@ -258,8 +299,8 @@ __device__ __forceinline__ u64 ll_word(unsigned payload, unsigned flag) {
 // It also follows the row that content was in at the leaf's start (corg),
 // which tells the other columns' interchanges their sources (swap_trsm.hip).
 // What bounds it: the chain A..D (1500-2100 cycles a column in one workgroup,
-// 4200 with 32, 945 of them the exchange's round trip), then E (4000-7000 a
-// group).  With several workgroups only the next group's columns are updated
+// 3700 with up to 16, 4700 with 32, 945 of them the exchange's round trip), then
+// E (4000-7000 a group).  With several workgroups only the next group's columns are updated
 // in E; each later step updates one further chunk while its exchange is in
 // flight.  Measured, 64 columns of FP64 (before: the whole row exchanged and
 // updated in every column, agent-scope stores): 512 rows 214 -> 95 us, 128
@@ -295,7 +336,7 @@ struct LeafLds {
 // content is in this thread's row now), zero_at (the first step with a zero
 // pivot, or -1).  PREF: a chunk's values of U are read while the one before
 // is applied.
-template <class T, int W, int NTH, bool MULTI, bool XCD0, bool PREF = true>
+template <class T, int W, int NTH, bool MULTI, bool XCD0, bool PREF = true, int DIRECT = 0>
 __device__ __forceinline__ void leaf_columns(T (&v)[W], LeafLds<T, W, NTH, MULTI>& S, int h, int w, int b, int G,
                                              unsigned tagbase, u64* xbuf, int* err, int& my_piv, int& corg,
                                              int& zero_at) {
@@ -340,7 +381,7 @@ __device__ __forceinline__ void leaf_columns(T (&v)[W], LeafLds<T, W, NTH, MULTI
   auto spin_check = [&](unsigned& spins) -> bool {
     __builtin_amdgcn_s_sleep(1);
     ++spins;
-    if ((spins & 255u) == 1u && ld_dev(err) != 0) return false;
+    if ((spins & 63u) == 0u && ld_dev(err) != 0) return false;  // (not in the first: a load more in every column)
     if (spins > (1u << 20)) {
       st_dev(err, 1);
       return false;
@@ -402,8 +443,19 @@ __device__ __forceinline__ void leaf_columns(T (&v)[W], LeafLds<T, W, NTH, MULTI
             S.rowk[par].osl = osl;
             S.rowk[par].org = corg;
           }
-          const unsigned wm = wave_max_recip(hi, v[kk], &rp);
+          // (DIRECT: the reciprocal after the key, while that is on its way)
+          const unsigned wm = DIRECT ? lanes_max<1, 64>(hi) : wave_max_recip(hi, v[kk], &rp);
           const int wl = pick_lane<T, 1, 64>(v[kk], cand, lr == k, hi, wm, &none);
+          if (DIRECT && lane == wl) {  // its key at once
+            u64* const kw = xbuf + (size_t)par * MSG_PAR + (b * NW + wave);
+            put(kw, (u64)direct_flag(flag, (none ? DIRECT_NONE : 0u) | (unsigned)osl << 6 | (unsigned)lane) << 32 |
+                        value_word(v[kk], VW - 1));
+            if (VW > 1) put(kw + DIRECT_CANDS, ll_word(value_word(v[kk], 0), flag));
+          }
+          if (DIRECT) {
+            rp = T(1) / v[kk];
+            asm volatile("" : "+v"(rp));  // (on all lanes, not in the one lane's branch)
+          }
           if (lane == wl) {
             typename L::Msg& ms = S.wmsg[par][wave];
 #pragma unroll
@@ -419,11 +471,91 @@ __device__ __forceinline__ void leaf_columns(T (&v)[W], LeafLds<T, W, NTH, MULTI
           wave_sync();
           if (lane < MW) mine = reinterpret_cast<const unsigned*>(&S.wmsg[par][wave])[lane];
         }
-        __syncthreads();
+        if (!DIRECT) __syncthreads();
         // ---- B, C
         int meta, porg;
         T uc[LG], rp;  // the pivot row's group values and its pivot's reciprocal (uniform)
-        if (MULTI) {
+        unsigned rk = 0;  // DIRECT: word `lane` of row k
+        if (DIRECT) {
+          const u64* const buf = xbuf + (size_t)par * MSG_PAR;
+          u64* const out = xbuf + (size_t)par * MSG_PAR + DIRECT_VALUES;
+          if (lane < MW) put(out + (b * NW + wave) * MW + lane, ll_word(mine, flag));
+          if (top_wave && lane < KW) {
+            const unsigned x = reinterpret_cast<const unsigned*>(&S.rowk[par])[lane];
+            put(xbuf + (size_t)par * MSG_PAR + DIRECT_ROWK + lane, ll_word(x, flag));
+          }
+          if (kk + 1 < W / LG && g > 0 && kk + 1 <= rest) {  // (as below)
+            T nl[LG], uu[LG];
+            load_u(uu, kk + 1);
+#pragma unroll
+            for (int i = 0; i < LG; ++i) nl[i] = -v[W - LG + i];
+            apply_u(uu, nl, v + LG * (kk + 1), k0);
+          }
+          // DIRECT candidates a lane: every wave folds them all
+          constexpr int CL = DIRECT > 0 ? DIRECT : 1;
+          const bool in = CL * lane < G * NW;  // (G * NW is a multiple of CL)
+          const u64* const pk = buf + (in ? CL * lane : 0);
+          const u64* const pr = buf + DIRECT_ROWK + (lane < KW ? lane : 0);
+          u64 x0[CL], x1[CL], x2;
+          unsigned spins = 0;
+          for (;;) {
+            bool miss = false;
+#pragma unroll
+            for (int q = 0; q < CL; ++q) {
+              x0[q] = ld_dev(pk + q);
+              x1[q] = VW > 1 ? ld_dev(pk + DIRECT_CANDS + q) : 0;
+            }
+            x2 = ld_dev(pr);
+#pragma unroll
+            for (int q = 0; q < CL; ++q)
+              miss |= (unsigned)(x0[q] >> 44) != direct_flag(flag, 0) >> 12 || (VW > 1 && (unsigned)(x1[q] >> 32) != flag);
+            miss |= (unsigned)(x2 >> 32) != flag;
+            if (failed || !__any(miss)) break;
+            if (!spin_check(spins)) {
+              failed = true;
+              S.fail = 1;
+              break;
+            }
+          }
+          rk = (unsigned)x2;
+          T cv = value_of<T>((unsigned)x0[0], (unsigned)x1[0]);
+          int cand = CL * lane;
+          unsigned km = (unsigned)(x0[0] >> 32) & 0xfffu;
+#pragma unroll
+          for (int q = 1; q < CL; ++q) {
+            const T ov = value_of<T>((unsigned)x0[q], (unsigned)x1[q]);
+            const unsigned om = (unsigned)(x0[q] >> 32) & 0xfffu;
+            const u64 ck = km & DIRECT_NONE ? 0ull : pivot_key(cv, cand * 64 + (int)(km & 63u) == k);
+            const u64 ok = om & DIRECT_NONE ? 0ull : pivot_key(ov, (CL * lane + q) * 64 + (int)(om & 63u) == k);
+            if (ok > ck) {
+              cv = ov;
+              km = om;
+              cand = CL * lane + q;
+            }
+          }
+          bool none;
+          const int wl = pick_lane<T, 1, 64>(cv, in && !(km & DIRECT_NONE), cand * 64 + (int)(km & 63u) == k, &none);
+          const int ws = __builtin_amdgcn_readlane(cand, wl);
+          // the winner's values and row
+          const u64* const pv = out + ws * MW + (lane < MW ? lane : 0);
+          u64 y;
+          for (;;) {
+            y = ld_dev(pv);
+            if (failed || !__any((unsigned)(y >> 32) != flag)) break;
+            if (!spin_check(spins)) {
+              failed = true;
+              S.fail = 1;
+              break;
+            }
+          }
+          const unsigned wm = (unsigned)__builtin_amdgcn_readlane((int)km, wl);
+          meta = (ws * 64 + (int)(wm & 63u)) | (int)(wm >> 6 & 31u) << 16;
+          porg = __builtin_amdgcn_readlane((int)(unsigned)y, (LG + 1) * VW + 1);
+#pragma unroll
+          for (int c = 0; c < LG; ++c) uc[c] = word_value<T>((int)(unsigned)y, VW * c);
+          rp = word_value<T>((int)(unsigned)y, VW * LG);
+          if (wave == NW - 1 && lane < LG * VW) reinterpret_cast<unsigned*>(S.l[kk])[lane] = (unsigned)y;
+        } else if (MULTI) {
           {
             const typename L::Msg& ms = S.wmsg[par][lane & (NW - 1)];
             const int cm = ms.meta;
@@ -544,11 +676,19 @@ __device__ __forceinline__ void leaf_columns(T (&v)[W], LeafLds<T, W, NTH, MULTI
             corg = porg;
           }
           if (p >= wrow0 && p < wrow0 + 64) {
+            T rv[LG];
+            int ro = 0, rg = 0;
+            if (DIRECT) {
+#pragma unroll
+              for (int c = 0; c < LG; ++c) rv[c] = word_value<T>((int)rk, VW * c);
+              ro = __builtin_amdgcn_readlane((int)rk, VW * LG);
+              rg = __builtin_amdgcn_readlane((int)rk, VW * LG + 1);
+            }
             if (lr == p) {
 #pragma unroll
-              for (int c = 0; c < LG; ++c) v[c] = S.rowk[par].v[c];
-              osl = S.rowk[par].osl;
-              corg = S.rowk[par].org;
+              for (int c = 0; c < LG; ++c) v[c] = DIRECT ? rv[c] : S.rowk[par].v[c];
+              osl = DIRECT ? ro : S.rowk[par].osl;
+              corg = DIRECT ? rg : S.rowk[par].org;
               if (myslot == NOSLOT) myslot = LG + kk;
             }
           }

@@ -535,7 +535,7 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
 
   // the panel's flag-in-data exchange needs a zeroed buffer per factorization;
   // the flag base starts over only long before it could wrap
-  if (c->leaf_tag > 0xF0000000u) c->leaf_tag = 0;
+  if (c->leaf_tag > 0x70000000u) c->leaf_tag = 0;
   launch_lu_init(reinterpret_cast<unsigned*>(xchg), panel_xchg_bytes(0) / sizeof(unsigned), err, fail > 0 ? 1 : 0, info,
                  s);
   mark(pa, fla, LA_PHASE_TRANSPOSE, 0);

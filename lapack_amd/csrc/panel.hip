@@ -48,7 +48,7 @@ template <> struct Sfmin<float> { static constexpr float v = 0x1p-126f; };
 __host__ __device__ __forceinline__ unsigned panel_xcds(int G) { return (unsigned)((G + 31) / 32); }
 
 // The leaf A(j0:m-1, j0:j0+w-1) in registers (leaf.h).
-template <class T, int W, int NTH, bool MULTI, bool XCD0>
+template <class T, int W, int NTH, bool MULTI, bool XCD0, int DIRECT = 0>
 __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, long ldt, int j0, int w, int m,
                                                         int* __restrict__ ipiv, int* __restrict__ info,
                                                         unsigned tagbase, u64* __restrict__ xbuf,
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
   // (the exchange's stores included) wherever the loop first reads v
   wait_vm();
   int my_piv, corg, zero_at;
-  leaf_columns<T, W, NTH, MULTI, XCD0>(v, S, h, w, b, G, tagbase, xbuf, err, my_piv, corg, zero_at);
+  leaf_columns<T, W, NTH, MULTI, XCD0, true, DIRECT>(v, S, h, w, b, G, tagbase, xbuf, err, my_piv, corg, zero_at);
   if (lr < h) {
     const int o = j0 + (corg >= 0 && corg < h ? corg : lr);  // (out of range only after a wait gave up)
     const int po = org.pin ? org.pin[o] : o;
@@ -338,13 +338,13 @@ static int launch_panel_t(T* Tm, long ldt, int j0, int w, int m, int* ipiv, int*
   if (h <= 0 || w <= 0) return 0;
   if (w > WMAX) return LA_ERR_LIMIT;
   u64* xb = reinterpret_cast<u64*>(xchg);
-#define LA_LEAF(W, NTH, MULTI, XCD0, blocks, g, ctr) \
-  getf2_leaf_kernel<T, W, NTH, MULTI, XCD0><<<blocks, NTH, 0, s>>>(Tm, ldt, j0, w, m, ipiv, info, tagbase, xb, err, g, ctr, \
-                                                              org)
+#define LA_LEAF(W, NTH, MULTI, XCD0, DIRECT, blocks, g, ctr) \
+  getf2_leaf_kernel<T, W, NTH, MULTI, XCD0, DIRECT><<<blocks, NTH, 0, s>>>(Tm, ldt, j0, w, m, ipiv, info, tagbase, xb, \
+                                                                      err, g, ctr, org)
   if (h <= 512) {
-    if (h <= 128) LA_LEAF(64, 128, false, false, 1, 1, nullptr);
-    else if (h <= 256) LA_LEAF(64, 256, false, false, 1, 1, nullptr);
-    else LA_LEAF(64, 512, false, false, 1, 1, nullptr);
+    if (h <= 128) LA_LEAF(64, 128, false, false, 0, 1, 1, nullptr);
+    else if (h <= 256) LA_LEAF(64, 256, false, false, 0, 1, 1, nullptr);
+    else LA_LEAF(64, 512, false, false, 0, 1, 1, nullptr);
     return 0;
   }
   const int G = (h + 511) / 512;
@@ -366,11 +366,18 @@ static int launch_panel_t(T* Tm, long ldt, int j0, int w, int m, int* ipiv, int*
     tall_org_kernel<<<1, 256, 0, s>>>(j0, kmax, m, ipiv, org);
     return 0;
   }
-  if (mode == PANEL_XCD0)
-    LA_LEAF(64, 512, true, true, (8 / (int)panel_xcds(G)) * G, G,
-            reinterpret_cast<unsigned*>(reinterpret_cast<char*>(xchg) + rank_offset()));
-  else
-    LA_LEAF(64, 512, true, false, G, G, nullptr);
+  unsigned* const ctr = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(xchg) + rank_offset());
+  const int direct = G <= 8 ? 1 : G <= 16 ? 2 : 0;
+  if (mode == PANEL_XCD0) {
+    const int blocks = (8 / (int)panel_xcds(G)) * G;
+    if (direct == 1) LA_LEAF(64, 512, true, true, 1, blocks, G, ctr);
+    else if (direct == 2) LA_LEAF(64, 512, true, true, 2, blocks, G, ctr);
+    else LA_LEAF(64, 512, true, true, 0, blocks, G, ctr);
+  } else {
+    if (direct == 1) LA_LEAF(64, 512, true, false, 1, G, G, nullptr);
+    else if (direct == 2) LA_LEAF(64, 512, true, false, 2, G, G, nullptr);
+    else LA_LEAF(64, 512, true, false, 0, G, G, nullptr);
+  }
 #undef LA_LEAF
   return 0;
 }
