@@ -155,11 +155,11 @@ int tune_plan(lapack_amd_batch_plan* p, hipStream_t s) {
 
 // Orders up to 512 take the register form, without a trial: it was faster than
 // the best of the panel forms for every batch measured.  Uniform orders,
-// best panel form -> register form, us:  FP64: 8 of 4..12 43 -> 33, 2000 of
-// 4..12 71 -> 64, 1000 of 16..64 197 -> 103, 3000 of 8..160 1233 -> 893, 4 of
-// 300..512 3447 -> 1797, 300 of 400..512 5977 -> 3714, 1000 of 100..256 1666 ->
-// 1472, 10000 of 16..512 62967 -> 32616.  FP32: 43 -> 31, 72 -> 68, 189 -> 118,
-// 983 -> 695, 3202 -> 1354, 5059 -> 1837, 1481 -> 858.
+// best panel form -> register form, us:  FP64: 8 of 4..12 43 -> 32, 2000 of
+// 4..12 71 -> 70, 1000 of 16..64 197 -> 107, 3000 of 8..160 1233 -> 845, 4 of
+// 300..512 3447 -> 1684, 300 of 400..512 5977 -> 3175, 1000 of 100..256 1666 ->
+// 1334, 10000 of 16..512 62967 -> 28238.  FP32: 43 -> 32, 72 -> 68, 189 -> 103,
+// 983 -> 645, 3202 -> 1344, 5059 -> 1858, 1481 -> 770.
 int default_cfg(int nmax, int elem) {
   if (nmax <= batched_leaf_nmax()) return LEAF_CFG;
   // Largest panel that fits, 256 threads (autotuning usually confirms NB 16 or 32).

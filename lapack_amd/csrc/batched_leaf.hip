@@ -26,7 +26,10 @@
 // Bound: per column the leaf's latency chain (about 2000 cycles; two
 // workgroups of 512 threads or more smaller ones on a CU overlap theirs), and
 // the trailing matrix read and written once per 32 columns (n^3/6 bytes per
-// matrix in FP64) where the batch exceeds the caches.
+// matrix in FP64) where the batch exceeds the caches.  10000 matrices of
+// order 16..512: 28.2 ms (best panel form 62.9); the substitution keeps 8 steps'
+// coefficients at a time and its rounds are not unrolled (32.6 ms with all of
+// them in flight: the registers then spilled).
 #include "leaf.h"
 #include "mfma.h"
 
@@ -42,6 +45,7 @@ constexpr int BW = 32;  // columns of a block
 template <class T, int K>
 __device__ __forceinline__ void unit_solve(T (&x)[2], T& t, const T (*sl)[BW + 1], int sub) {
   if constexpr (K < BW) {
+    if constexpr (K % 8 == 0) asm volatile("" ::: "memory");  // (coefficients of 8 steps in flight, not of all)
     constexpr int KM = K / 16, KS = K % 16;
     T y = x[KM];
     fmac_from<KS>(y, x[KM], sl[K][16 * KM + sub]);
@@ -146,7 +150,7 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4))) void g
             s_x[e & (BW - 1)][e / BW] = g[u];
           }
           __syncthreads();
-#pragma unroll
+#pragma unroll 1
           for (int q = 0; q < CB; q += NTH / 16) {
             const int c = q + te / 16;
             T x[2] = {s_x[li][c], s_x[16 + li][c]}, t;
@@ -164,6 +168,7 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4))) void g
           if (below) {
             const int nct = min(CB, n - cb + 15) / 16;
             const long lo = (long)MM::row(lk, 0) * lda;
+#pragma unroll 1
             for (int rp = 64 * wave < BW ? BW / 32 : 0; rp < 2; ++rp) {
               T a[2][BW / 4];
               long src[2];
@@ -175,6 +180,7 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4))) void g
 #pragma unroll
                 for (int s = 0; s < BW / 4; ++s) a[rt][s] = (A + (long)(k0 + 4 * s) * lda)[o];
               }
+#pragma unroll 1
               for (int ct = 0; ct < nct; ++ct) {
                 // a lane's columns are MM::row(lk, r) past the tile's first;
                 // past the matrix it reads and writes nothing
