@@ -1011,7 +1011,7 @@ static int update_dma() {
 // (LAPACK_AMD_UPD_DMA_KS, 16 or 32, default 32; read at every launch).
 // Alone 32 is 1-2 % slower (107.3 against 109.3 TFLOP/s at m = n = 16128),
 // beside the panel faster: SGETRF 95.2 -> 90.3 ms at n = 16384, 314.2 ->
-// 311.7 ms at n = 32768 (the panel's boundary launches wait less).
+// 311.7 ms at n = 32768 (the panel's own launches wait less).
 static int update_dma_ks() {
   const char* e = std::getenv("LAPACK_AMD_UPD_DMA_KS");
   return (e && *e) ? std::atoi(e) : 32;
