@@ -47,46 +47,52 @@ __device__ __forceinline__ long m_index(int i, int c, long lda) {
   return TRANS ? (long)c + (long)i * lda : (long)i + (long)c * lda;
 }
 
-// Replaces the TB x TB triangle in sD (NTH threads; unit diagonal when
-// UNIT) by its inverse, by doubling: the 1x1 blocks are the reciprocals of
-// the diagonal (1 when unit); then for b = 1, 2, .., 32 every pair of
-// inverted b x b diagonal blocks A (first) and B (second) gets its
-// off-diagonal block, -inv(B) C inv(A) below the diagonal (lower M) or
-// -inv(A) C inv(B) above it (upper M), through a b x b temporary tmp
-// (>= TB*TB/4 values).  Ends with a barrier.
-template <class T, bool LOWERM, bool UNIT, int NTH = 256>
-__device__ void invert_diag(T (*sD)[TB + 1], T* tmp) {
-  const int tid = threadIdx.x;
-  if (tid < TB) sD[tid][tid] = UNIT ? T(1) : T(1) / sD[tid][tid];
+// Replaces the TB x TB triangle in sD (256 threads; unit diagonal when UNIT, the
+// other triangle zero) by its inverse V, in the order of the substitution and by
+// 16 x 16 blocks: the diagonal ones by substitution, 16 lanes a column; then, block
+// column j = 2, 1, 0, V(i, j) = -sum over k = j+1 .. i of V(i, k) (M(k, j) V(j, j)) on the
+// matrix cores, a block a wave.  (Doubling through LDS took 15 us of a sweep.)
+// tmp: 3 * 16 * 17 values.  Ends with a barrier.
+template <class T, bool LOWERM, bool UNIT>
+__device__ __forceinline__ void invert_diag(T (*sD)[TB + 1], T* tmp) {
+  typedef Mfma<T> MM;
+  typedef typename MM::acc_t acc_t;
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto E = [&](int i, int k) -> T& { return LOWERM ? sD[i][k] : sD[TB - 1 - i][TB - 1 - k]; };
+  T xs[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    T x = li == tid / 16 ? T(1) : T(0);
+    const T r = UNIT ? T(1) : T(1) / E(16 * m + li, 16 * m + li);
+    diag_steps<T, UNIT ? DIAG_UNIT : DIAG_MULTIPLY, 0>(
+        x, r, [&](int k) { return li > k ? -E(16 * m + li, 16 * m + k) : T(0); });
+    xs[m] = x;
+  }
   __syncthreads();
-  for (int bsz = 1; bsz < TB; bsz *= 2) {
-    const int cnt = (TB / (2 * bsz)) * bsz * bsz;  // elements of all pairs' blocks
-    // phase 1: tmp = C inv(A) (lower) or inv(A) C (upper), per pair
-    for (int e = tid; e < cnt; e += NTH) {
-      const int pr = e / (bsz * bsz), r = (e / bsz) % bsz, c = e % bsz;
-      const int a0 = 2 * pr * bsz, b0 = a0 + bsz;
-      T acc = T(0);
-      if (LOWERM) {
-        for (int k = c; k < bsz; ++k) acc = acc + sD[b0 + r][a0 + k] * sD[a0 + k][a0 + c];
-      } else {
-        for (int k = r; k < bsz; ++k) acc = acc + sD[a0 + r][a0 + k] * sD[a0 + k][b0 + c];
-      }
-      tmp[e] = acc;
+#pragma unroll
+  for (int m = 0; m < 4; ++m) E(16 * m + li, 16 * m + tid / 16) = xs[m];
+  __syncthreads();
+#pragma unroll 1
+  for (int j = 2; j >= 0; --j) {
+    const int i = j + 1 + wave;  // this wave's block of the column
+    if (i < 4) {
+      acc_t acc = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+      for (int s = 0; s < 16; s += 4) acc = MM::op(E(16 * i + li, 16 * j + s + lk), E(16 * j + s + lk, 16 * j + li), acc);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tmp[(wave * 16 + MM::row(lk, r)) * 17 + li] = acc[r];
     }
     __syncthreads();
-    // phase 2: off-diagonal block = -inv(B) tmp (lower) or -tmp inv(B) (upper)
-    for (int e = tid; e < cnt; e += NTH) {
-      const int pr = e / (bsz * bsz), r = (e / bsz) % bsz, c = e % bsz;
-      const int a0 = 2 * pr * bsz, b0 = a0 + bsz;
-      const T* tp = tmp + (size_t)pr * bsz * bsz;
-      T acc = T(0);
-      if (LOWERM) {
-        for (int k = 0; k <= r; ++k) acc = acc + sD[b0 + r][b0 + k] * tp[k * bsz + c];
-        sD[b0 + r][a0 + c] = -acc;
-      } else {
-        for (int k = 0; k <= c; ++k) acc = acc + tp[r * bsz + k] * sD[b0 + k][b0 + c];
-        sD[a0 + r][b0 + c] = -acc;
-      }
+    if (i < 4) {
+      acc_t acc = {T(0), T(0), T(0), T(0)};
+#pragma unroll 1
+      for (int k = j + 1; k <= i; ++k)
+#pragma unroll
+        for (int s = 0; s < 16; s += 4)
+          acc = MM::op(E(16 * i + li, 16 * k + s + lk), tmp[((k - j - 1) * 16 + s + lk) * 17 + li], acc);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) E(16 * i + MM::row(lk, r), 16 * j + li) = -acc[r];
     }
     __syncthreads();
   }

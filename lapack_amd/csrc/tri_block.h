@@ -47,6 +47,18 @@ __device__ __forceinline__ void tri_step(T (&x)[4], const T (&d)[4], const T (&r
   }
 }
 
+// Steps K .. 15 of the substitution in one 16 x 16 block, its coefficients -M(i, k)
+// at c(k) of the lane's row.
+template <class T, Diag D, int K, class C>
+__device__ __forceinline__ void diag_steps(T& x, T r, C c) {
+  if constexpr (K < 16) {
+    fmac_from<K>(x, by_diag<T, D>(x, r, r), c(K));
+    diag_steps<T, D, K + 1>(x, r, c);
+  } else {
+    x = by_diag<T, D>(x, r, r);
+  }
+}
+
 // Sub-blocks m_lo .. m_hi - 1 (the others hold rows past the matrix).
 template <class T, Diag D>
 __device__ __forceinline__ void tri_solve(T (&x)[4], const T (&d)[4], const T (&r)[4], const TriBlock<T>& tri, int sub,

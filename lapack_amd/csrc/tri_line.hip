@@ -64,17 +64,6 @@ __device__ __forceinline__ T dot16(const T (&m)[16], T x) {
   return p0 + p1;
 }
 
-// Steps K .. 15 of the substitution in one 16 x 16 block.
-template <class T, Diag D, int K>
-__device__ __forceinline__ void diag_steps(T& x, T r, const T (*c)[17], int sub) {
-  if constexpr (K < 16) {
-    fmac_from<K>(x, by_diag<T, D>(x, r, r), c[K][sub]);
-    diag_steps<T, D, K + 1>(x, r, c, sub);
-  } else {
-    x = by_diag<T, D>(x, r, r);
-  }
-}
-
 // Sum over the 16 lanes of a row, in every lane.
 template <int ROR>
 __device__ __forceinline__ double ror16(double v) {
@@ -122,7 +111,8 @@ __device__ __forceinline__ void invert_triangles(LineLds<T>& S, int tid) {
     const int m = wave >> 2, j = tid / 16 & 15;  // block m, column j
     T x = li == j ? T(1) : T(0);
     const T r = UNIT ? T(1) : S.rec[64 * blk + at(16 * m + li)];
-    diag_steps<T, UNIT ? DIAG_UNIT : DIAG_MULTIPLY, 0>(x, r, S.tri[blk].c[m * (m + 1) / 2 + m], li);
+    const auto* const c = S.tri[blk].c[m * (m + 1) / 2 + m];
+    diag_steps<T, UNIT ? DIAG_UNIT : DIAG_MULTIPLY, 0>(x, r, [&](int k) { return c[k][li]; });
     S.inv[blk][at(16 * m + li)][at(16 * m + j)] = x;
   }
 #pragma unroll 1
