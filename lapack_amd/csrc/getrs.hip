@@ -20,9 +20,9 @@
 //     the one finished most recently -- gets a round of its own, so the
 //     work left once it arrives is one tile;
 //   * before its dependencies arrive, the workgroup inverts the 64x64
-//     diagonal block in LDS (doubling over 2x2 block-triangular inverses),
-//     so that once they have arrived the block costs a 64-term product per
-//     row, not a 64-step chain;
+//     diagonal block in LDS (16 x 16 blocks, then products with them), so
+//     that once they have arrived the block costs a 64-term product per row,
+//     not a 64-step chain;
 //   * the four partial sums per row are added in LDS, y = b + acc, and
 //     x = inv(M_dd) y, one wavefront per four right-hand sides;
 //   * x is stored with device-coherent stores, the stores are waited for,
@@ -63,11 +63,9 @@ __device__ __forceinline__ void invert_diag(T (*sD)[TB + 1], T* tmp) {
   T xs[4];
 #pragma unroll
   for (int m = 0; m < 4; ++m) {
-    T x = li == tid / 16 ? T(1) : T(0);
     const T r = UNIT ? T(1) : T(1) / E(16 * m + li, 16 * m + li);
-    diag_steps<T, UNIT ? DIAG_UNIT : DIAG_MULTIPLY, 0>(
-        x, r, [&](int k) { return li > k ? -E(16 * m + li, 16 * m + k) : T(0); });
-    xs[m] = x;
+    xs[m] = diag_inverse<T, UNIT ? DIAG_UNIT : DIAG_MULTIPLY>(
+        r, li, tid / 16, [&](int k) { return li > k ? -E(16 * m + li, 16 * m + k) : T(0); });
   }
   __syncthreads();
 #pragma unroll

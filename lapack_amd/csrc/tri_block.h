@@ -47,16 +47,25 @@ __device__ __forceinline__ void tri_step(T (&x)[4], const T (&d)[4], const T (&r
   }
 }
 
-// Steps K .. 15 of the substitution in one 16 x 16 block, its coefficients -M(i, k)
-// at c(k) of the lane's row.
+// Column j of the inverse of one 16 x 16 block by substitution, K the next step:
+// lane sub of 16 holds row sub, the reciprocal r of its diagonal and, at c(k), the
+// coefficients -M(sub, k), zero for k >= sub.  A lane keeps its value from its own step:
+// the later products with zero would turn it into a NaN where a diagonal is zero
+// and the steps are infinite, and so would a zero above the diagonal times r.
 template <class T, Diag D, int K, class C>
-__device__ __forceinline__ void diag_steps(T& x, T r, C c) {
+__device__ __forceinline__ void diag_steps(T& own, T x, T r, int sub, C c) {
   if constexpr (K < 16) {
-    fmac_from<K>(x, by_diag<T, D>(x, r, r), c(K));
-    diag_steps<T, D, K + 1>(x, r, c);
-  } else {
-    x = by_diag<T, D>(x, r, r);
+    const T q = by_diag<T, D>(x, r, r);
+    own = sub == K ? q : own;
+    if constexpr (K < 15) fmac_from<K>(x, q, c(K));
+    diag_steps<T, D, K + 1>(own, x, r, sub, c);
   }
+}
+template <class T, Diag D, class C>
+__device__ __forceinline__ T diag_inverse(T r, int sub, int j, C c) {
+  T own = T(0);
+  diag_steps<T, D, 0>(own, sub == j ? T(1) : T(0), sub >= j ? r : T(0), sub, c);
+  return own;
 }
 
 // Sub-blocks m_lo .. m_hi - 1 (the others hold rows past the matrix).

@@ -109,11 +109,10 @@ __device__ __forceinline__ void invert_triangles(LineLds<T>& S, int tid) {
 #pragma unroll 1
   for (int blk = 0; blk < 2; ++blk) {
     const int m = wave >> 2, j = tid / 16 & 15;  // block m, column j
-    T x = li == j ? T(1) : T(0);
     const T r = UNIT ? T(1) : S.rec[64 * blk + at(16 * m + li)];
     const auto* const c = S.tri[blk].c[m * (m + 1) / 2 + m];
-    diag_steps<T, UNIT ? DIAG_UNIT : DIAG_MULTIPLY, 0>(x, r, [&](int k) { return c[k][li]; });
-    S.inv[blk][at(16 * m + li)][at(16 * m + j)] = x;
+    S.inv[blk][at(16 * m + li)][at(16 * m + j)] =
+        diag_inverse<T, UNIT ? DIAG_UNIT : DIAG_MULTIPLY>(r, li, j, [&](int k) { return c[k][li]; });
   }
 #pragma unroll 1
   for (int d = 1; d < 4; ++d) {

@@ -76,3 +76,31 @@ def test_gesv_solves_only_the_nonsingular(dev, n, nrhs):
         else:
             assert info == 0
             assert oracle.dget02(np.asfortranarray(m), np.asfortranarray(x), np.asfortranarray(b)) < 30.0
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("nrhs", [1, 3, 16])
+@pytest.mark.parametrize("n,zero", [(5, 2), (16, 15), (16, 0), (64, 40), (100, 55), (130, 66), (200, 199), (300, 150)])
+def test_zero_on_the_diagonal(dev, n, zero, nrhs, dtype):
+    """Factors with a zero on U's diagonal: what the substitution solves before it
+    reaches the zero is not touched by it (BLAS/SRC/dtrsm.f:277-300), the row of the
+    zero is not finite.  (Against A^T the second sweep takes it to every row.)"""
+    dbl = dtype == np.float64
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((n, n)) + 4.0 * np.sqrt(n) * np.eye(n)
+    lu = (oracle.dgetrf if dbl else oracle.sgetrf)(np.asfortranarray(a.astype(dtype)))[0]
+    lu[zero, zero] = 0
+    p = np.arange(1, n + 1, dtype=np.int32)  # (rows stay in place)
+    b = rng.standard_normal((n, nrhs)).astype(dtype)
+    d_a, d_p = torch.from_numpy(np.ascontiguousarray(lu.T)).cuda(), torch.from_numpy(p).cuda()
+    l, u = np.tril(lu.astype(np.float64), -1) + np.eye(n), np.triu(lu.astype(np.float64))
+    tol = 64 * n * (2.0 ** -53 if dbl else 2.0 ** -24)
+    d_b = torch.from_numpy(b.T.copy()).cuda()
+    assert (la.dgetrs_async if dbl else la.sgetrs_async)("N", n, nrhs, d_a, n, d_p, d_b, n) == 0
+    torch.cuda.synchronize()
+    assert la.device_status() == 0
+    x = d_b.cpu().numpy().T
+    ref = np.linalg.solve(u[zero + 1:, zero + 1:], np.linalg.solve(l, b)[zero + 1:])
+    assert not np.isfinite(x[zero]).any()
+    if zero + 1 < n:
+        assert np.abs(x[zero + 1:] - ref).max() <= tol * np.abs(ref).max()
