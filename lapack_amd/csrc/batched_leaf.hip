@@ -59,6 +59,20 @@ __device__ __forceinline__ void unit_solve(T (&x)[2], T& t, const T (*sl)[BW + 1
   }
 }
 
+// The same with DTRSM's test: a zero of the solution is not multiplied
+// (BLAS/SRC/dtrsm.f:177-190), which matters where L is not finite.
+template <class T>
+__device__ __forceinline__ void unit_solve_tested(T (&x)[2], const T (*sl)[BW + 1], int lane, int sub) {
+#pragma unroll 1
+  for (int k = 0; k < BW; ++k) {
+    const T xk = __shfl(k < 16 ? x[0] : x[1], (lane & 48) | (k & 15));
+    if (xk != T(0)) {
+      if (sub > k) x[0] = x[0] + xk * sl[k][sub];
+      if (16 + sub > k) x[1] = x[1] + xk * sl[k][16 + sub];
+    }
+  }
+}
+
 template <class T, int NTH>
 __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4))) void getrf_batched_leaf_kernel(int first, int last, const int* __restrict__ nv,
                                                                     T* const* __restrict__ av,
@@ -155,6 +169,12 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4))) void g
             const int c = q + te / 16;
             T x[2] = {s_x[li][c], s_x[16 + li][c]}, t;
             unit_solve<T, 0>(x, t, s_l, li);
+            // (an L that is not finite shows in every column's result)
+            if (__builtin_expect(__any(!__builtin_isfinite(x[0]) || !__builtin_isfinite(x[1])), 0)) {
+              x[0] = s_x[li][c];
+              x[1] = s_x[16 + li][c];
+              unit_solve_tested(x, s_l, le, li);
+            }
             s_x[li][c] = x[0];
             s_x[16 + li][c] = x[1];
           }

@@ -73,3 +73,39 @@ def test_register_form(dev, kind, dtype):
             assert p[0] == p_r[0] == p_old[0] == 1
             assert (np.abs(np.tril(lu, -1)) <= 1.0).all()
         assert oracle.dget01(a, lu, p[:n]) * scale < THRESH, (kind, n)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["nan_below_the_head", "two_infinities"])
+def test_zeros_right_of_a_block_that_is_not_finite(dev, kind, dtype):
+    """DTRSM does not multiply a zero of the solution (BLAS/SRC/dtrsm.f:177-190):
+    where L is not finite, a column right of the block whose rows of U are zero
+    keeps them.  Infinities and NaNs lie where the panel form with blocks of the
+    same 32 columns has them, IPIV and INFO are its."""
+    ns = [33, 34, 48, 65, 100, 129, 200, 257, 300, 512]
+    bt = Batch(ns, [1] * len(ns), 47, dtype)
+    for k, (n, l, o) in enumerate(zip(ns, bt.ldas, bt.aoff)):
+        a = bt.h_a[o:o + n * l].reshape(n, l)  # a[c, r] = A(r, c)
+        if kind == "nan_below_the_head":
+            a[3, n - 2] = np.nan
+            a[7, 20] = np.nan
+        else:  # the first becomes the pivot, the second's multiplier is inf / inf
+            a[2, n // 2] = np.inf
+            a[2, n - 1] = -np.inf
+        for c in range(32, n, 3):  # columns of zeros, and of zeros in the first rows
+            a[c, :n if c % 2 else min(n, 40)] = 0.0
+    bt.d_a0.copy_(torch.from_numpy(bt.h_a))
+    plan = la.BatchPlan(ns, "d" if dtype == np.float64 else "s", autotune=False)
+    assert plan.set_config(32, 512) == 0
+    lu_all, piv_all, info_all = factor(bt, plan)
+    assert plan.set_config(32, 256) == 0
+    old_all, oldp_all, oldi_all = factor(bt, plan)
+    np.testing.assert_array_equal(info_all, oldi_all)
+    for k, n in enumerate(ns):
+        s = slice(k * bt.nmax, k * bt.nmax + n)
+        np.testing.assert_array_equal(piv_all[s], oldp_all[s], err_msg=str(n))
+        lu, old = bt.a_host(k, lu_all), bt.a_host(k, old_all)
+        zero_rows = (old[:32, 32:] == 0).any()
+        assert np.isnan(old[:, :32]).any() and zero_rows, n
+        np.testing.assert_array_equal(np.isnan(lu), np.isnan(old), err_msg=str(n))
+        np.testing.assert_array_equal(np.isinf(lu), np.isinf(old), err_msg=str(n))
