@@ -48,52 +48,76 @@ __device__ __forceinline__ long m_index(int i, int c, long lda) {
 }
 
 // Replaces the TB x TB triangle in sD (256 threads; unit diagonal when UNIT, the
-// other triangle zero) by its inverse V, in the order of the substitution and by
-// 16 x 16 blocks: the diagonal ones by substitution, 16 lanes a column; then, block
-// column j = 2, 1, 0, V(i, j) = -sum over k = j+1 .. i of V(i, k) (M(k, j) V(j, j)) on the
-// matrix cores, a block a wave.  (Doubling through LDS took 15 us of a sweep.)
+// other triangle zero) by its inverse V (tri_block.h): the 16 x 16 blocks of the
+// diagonal, then a wave per block column (LOWERM; wave j) or block row (wave 3 - i),
+// which needs nobody else's: M's blocks in registers before V replaces them.
+// (Doubling through LDS took 15 us of a sweep.)
 // tmp: 3 * 16 * 17 values.  Ends with a barrier.
 template <class T, bool LOWERM, bool UNIT>
 __device__ __forceinline__ void invert_diag(T (*sD)[TB + 1], T* tmp) {
   typedef Mfma<T> MM;
   typedef typename MM::acc_t acc_t;
+  constexpr Diag D = UNIT ? DIAG_UNIT : DIAG_MULTIPLY;
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   auto E = [&](int i, int k) -> T& { return LOWERM ? sD[i][k] : sD[TB - 1 - i][TB - 1 - k]; };
   T xs[4];
 #pragma unroll
   for (int m = 0; m < 4; ++m) {
-    const T r = UNIT ? T(1) : T(1) / E(16 * m + li, 16 * m + li);
-    xs[m] = diag_inverse<T, UNIT ? DIAG_UNIT : DIAG_MULTIPLY>(
-        r, li, tid / 16, [&](int k) { return li > k ? -E(16 * m + li, 16 * m + k) : T(0); });
+    const int o = 16 * m;
+    if constexpr (LOWERM) {
+      const T r = UNIT ? T(1) : T(1) / E(o + li, o + li);
+      xs[m] = diag_inverse<T, D>(r, li, tid / 16, [&](int k) { return li > k ? -E(o + li, o + k) : T(0); });
+    } else {
+      const T r = UNIT ? T(1) : T(1) / E(o + 15 - li, o + 15 - li);
+      xs[m] = diag_inverse_row<T, D>(r, li, tid / 16, [&](int a, int b) { return a > b ? -E(o + a, o + b) : T(0); });
+    }
   }
+  // M's blocks: [d - 1][z] is M(wave + d, wave + z), or M(3 - wave - d + 1 + z, 3 - wave - d)
+  T mb[3][3][4];
+#pragma unroll
+  for (int d = 1; d < 4; ++d)
+#pragma unroll
+    for (int z = 0; z < d; ++z)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (wave + d < 4)
+          mb[d - 1][z][s] = LOWERM ? -E(16 * (wave + d) + li, 16 * (wave + z) + 4 * s + lk)
+                                   : -E(16 * (4 - wave - d + z) + 4 * s + lk, 16 * (3 - wave - d) + li);
   __syncthreads();
 #pragma unroll
-  for (int m = 0; m < 4; ++m) E(16 * m + li, 16 * m + tid / 16) = xs[m];
-  __syncthreads();
-#pragma unroll 1
-  for (int j = 2; j >= 0; --j) {
-    const int i = j + 1 + wave;  // this wave's block of the column
-    if (i < 4) {
-      acc_t acc = {T(0), T(0), T(0), T(0)};
-#pragma unroll
-      for (int s = 0; s < 16; s += 4) acc = MM::op(E(16 * i + li, 16 * j + s + lk), E(16 * j + s + lk, 16 * j + li), acc);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) tmp[(wave * 16 + MM::row(lk, r)) * 17 + li] = acc[r];
-    }
-    __syncthreads();
-    if (i < 4) {
-      acc_t acc = {T(0), T(0), T(0), T(0)};
-#pragma unroll 1
-      for (int k = j + 1; k <= i; ++k)
-#pragma unroll
-        for (int s = 0; s < 16; s += 4)
-          acc = MM::op(E(16 * i + li, 16 * k + s + lk), tmp[((k - j - 1) * 16 + s + lk) * 17 + li], acc);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) E(16 * i + MM::row(lk, r), 16 * j + li) = -acc[r];
-    }
-    __syncthreads();
+  for (int m = 0; m < 4; ++m) {
+    if (LOWERM) E(16 * m + li, 16 * m + tid / 16) = xs[m];
+    else E(16 * m + tid / 16, 16 * m + 15 - li) = xs[m];
   }
+  __syncthreads();
+  T* const t = tmp + wave * 16 * 17;
+#pragma unroll
+  for (int d = 1; d < 4; ++d) {
+    if (wave + d < 4) {
+      const int i = LOWERM ? wave + d : 3 - wave, j = LOWERM ? wave : 3 - wave - d;
+      acc_t acc = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+      for (int z = 0; z < d; ++z) {
+        const int k = LOWERM ? j + z : j + 1 + z;
+        acc = acc + (LOWERM ? product16<T>([&](int s) { return mb[d - 1][z][s / 4]; },
+                                           [&](int s) { return E(16 * k + s + lk, 16 * j + li); })
+                            : product16<T>([&](int s) { return E(16 * i + li, 16 * k + s + lk); },
+                                           [&](int s) { return mb[d - 1][z][s / 4]; }));
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t[MM::row(lk, r) * 17 + li] = acc[r];
+      wave_sync();
+      acc = LOWERM ? product16<T>([&](int s) { return E(16 * i + li, 16 * i + s + lk); },
+                                  [&](int s) { return t[(s + lk) * 17 + li]; })
+                   : product16<T>([&](int s) { return t[li * 17 + s + lk]; },
+                                  [&](int s) { return E(16 * j + s + lk, 16 * j + li); });
+#pragma unroll
+      for (int r = 0; r < 4; ++r) E(16 * i + MM::row(lk, r), 16 * j + li) = acc[r];
+      wave_sync();
+    }
+  }
+  __syncthreads();
 }
 
 // QN: right-hand sides handled per launch (4 or 16).  Reads the

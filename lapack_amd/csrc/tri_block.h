@@ -4,6 +4,7 @@
 // are still to come.
 #pragma once
 #include "leaf.h"
+#include "mfma.h"
 
 namespace la {
 
@@ -66,6 +67,35 @@ __device__ __forceinline__ T diag_inverse(T r, int sub, int j, C c) {
   T own = T(0);
   diag_steps<T, D, 0>(own, sub == j ? T(1) : T(0), sub >= j ? r : T(0), sub, c);
   return own;
+}
+
+// ---- the inverse V of a triangle M by 16 x 16 blocks, in the order of the substitution ----
+// Which of V's two residuals is the small one, and so the error of x = V y, follows
+// from the order of its products.  By columns, V(i, j) = V(i, i) sum -M(i, k) V(k, j),
+// is the better one where M's rows are solved downwards (lower M), by rows, V(i, j) =
+// (sum V(i, k) -M(k, j)) V(j, j), where they are solved upwards.  Every product of 16
+// terms runs in two chains.  Error of V against doubling by 2 x 2 block triangles (64 rows, LU
+// factors of N(0,1) matrices): 0.94 to 0.97; all four triangles by columns 0.95 to
+// 1.24, -sum V(i, k) (M(k, j) V(j, j)) 1.07 to 1.45.
+
+// Row j of the inverse of one 16 x 16 block: column 15 - j of the inverse of its
+// mirror image P(a, b) = M(15 - b, 15 - a).  Lane sub of 16 gets V(j, 15 - sub); r
+// is the reciprocal of M's diagonal 15 - sub, c(a, b) is -M(a, b), zero for a <= b.
+template <class T, Diag D, class C>
+__device__ __forceinline__ T diag_inverse_row(T r, int sub, int j, C c) {
+  return diag_inverse<T, D>(r, sub, 15 - j, [&](int k) { return c(15 - k, 15 - sub); });
+}
+
+// The product of two 16 x 16 blocks on the matrix cores; lane (li, lk) gives
+// A(li, s + lk) and B(s + lk, li) for s = 0, 4, 8, 12.
+template <class T, class FA, class FB>
+__device__ __forceinline__ typename Mfma<T>::acc_t product16(FA a, FB b) {
+  typedef Mfma<T> MM;
+  const typename MM::acc_t zero = {T(0), T(0), T(0), T(0)};
+  typename MM::acc_t p = MM::op(a(0), b(0), zero), q = MM::op(a(4), b(4), zero);
+  p = MM::op(a(8), b(8), p);
+  q = MM::op(a(12), b(12), q);
+  return p + q;
 }
 
 // Sub-blocks m_lo .. m_hi - 1 (the others hold rows past the matrix).

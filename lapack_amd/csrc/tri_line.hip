@@ -96,23 +96,27 @@ struct LineLds {
   int t, failed;
 };
 
-// The inverses of both triangles into S.inv, which holds zeros.  V in the order
-// of the substitution, by 16 x 16 blocks: V(i, i) by substitution, 16 lanes a
-// column; V(i, j) = V(i, i) sum over k = j .. i-1 of -M(i, k) V(k, j), the blocks
-// of equal i - j at once, a wave each.
+// The inverses of both triangles into S.inv, which holds zeros (tri_block.h): the
+// 16 x 16 blocks of the diagonal, then the blocks of equal i - j at once, a wave each.
 template <class T, bool LOWERM, bool UNIT>
 __device__ __forceinline__ void invert_triangles(LineLds<T>& S, int tid) {
   typedef Mfma<T> MM;
+  constexpr Diag D = UNIT ? DIAG_UNIT : DIAG_MULTIPLY;
   const int lane = tid & 63, li = lane & 15, lk = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   auto at = [](int i) { return LOWERM ? i : 63 - i; };
 #pragma unroll 1
   for (int blk = 0; blk < 2; ++blk) {
-    const int m = wave >> 2, j = tid / 16 & 15;  // block m, column j
-    const T r = UNIT ? T(1) : S.rec[64 * blk + at(16 * m + li)];
+    const int m = wave >> 2, j = tid / 16 & 15;  // block m, column (LOWERM) or row j
     const auto* const c = S.tri[blk].c[m * (m + 1) / 2 + m];
-    S.inv[blk][at(16 * m + li)][at(16 * m + j)] =
-        diag_inverse<T, UNIT ? DIAG_UNIT : DIAG_MULTIPLY>(r, li, j, [&](int k) { return c[k][li]; });
+    if constexpr (LOWERM) {
+      const T r = UNIT ? T(1) : S.rec[64 * blk + at(16 * m + li)];
+      S.inv[blk][at(16 * m + li)][at(16 * m + j)] = diag_inverse<T, D>(r, li, j, [&](int k) { return c[k][li]; });
+    } else {
+      const T r = UNIT ? T(1) : S.rec[64 * blk + at(16 * m + 15 - li)];
+      S.inv[blk][at(16 * m + j)][at(16 * m + 15 - li)] =
+          diag_inverse_row<T, D>(r, li, j, [&](int a, int b) { return c[b][a]; });
+    }
   }
 #pragma unroll 1
   for (int d = 1; d < 4; ++d) {
@@ -120,21 +124,25 @@ __device__ __forceinline__ void invert_triangles(LineLds<T>& S, int tid) {
     const int cnt = 4 - d;
     if (wave < 2 * cnt) {
       const int blk = wave >= cnt, j = wave - blk * cnt, i = j + d;
+      T(*const tmp)[17] = S.tmp[wave];
+      auto V = [&](int r, int q, int a, int b) -> T& { return S.inv[blk][at(16 * r + a)][at(16 * q + b)]; };
+      auto C = [&](int r, int q, int a, int b) { return S.tri[blk].c[r * (r + 1) / 2 + q][b][a]; };
       typename MM::acc_t acc = {T(0), T(0), T(0), T(0)};
 #pragma unroll 1
-      for (int k = j; k < i; ++k)
-#pragma unroll
-        for (int s = 0; s < 16; s += 4)
-          acc = MM::op(S.tri[blk].c[i * (i + 1) / 2 + k][s + lk][li], S.inv[blk][at(16 * k + s + lk)][at(16 * j + li)], acc);
-      T(*const tmp)[17] = S.tmp[wave];
+      for (int z = 0; z < d; ++z) {
+        const int k = LOWERM ? j + z : j + 1 + z;
+        acc = acc + (LOWERM ? product16<T>([&](int s) { return C(i, k, li, s + lk); },
+                                           [&](int s) { return V(k, j, s + lk, li); })
+                            : product16<T>([&](int s) { return V(i, k, li, s + lk); },
+                                           [&](int s) { return C(k, j, s + lk, li); }));
+      }
 #pragma unroll
       for (int r = 0; r < 4; ++r) tmp[MM::row(lk, r)][li] = acc[r];
       wave_sync();
-      acc = {T(0), T(0), T(0), T(0)};
+      acc = LOWERM ? product16<T>([&](int s) { return V(i, i, li, s + lk); }, [&](int s) { return tmp[s + lk][li]; })
+                   : product16<T>([&](int s) { return tmp[li][s + lk]; }, [&](int s) { return V(j, j, s + lk, li); });
 #pragma unroll
-      for (int s = 0; s < 16; s += 4) acc = MM::op(S.inv[blk][at(16 * i + li)][at(16 * i + s + lk)], tmp[s + lk][li], acc);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S.inv[blk][at(16 * i + MM::row(lk, r))][at(16 * j + li)] = acc[r];
+      for (int r = 0; r < 4; ++r) V(i, j, MM::row(lk, r), li) = acc[r];
     }
   }
   __syncthreads();
