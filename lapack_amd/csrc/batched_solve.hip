@@ -28,8 +28,12 @@
 // of order 16..512 1718 / 3033.  (One wave for orders up to 64 was no faster:
 // 3000 of order 8..64 72 us against 70.)  Against one wave per block of rows,
 // 64-step substitutions by shuffles and interchanges by one lane: 10000 solves
-// of order 16..512 4700 -> 1720 us, the 256 adjoints 6420 -> 1174 (650 of them
+// of order 16..512 4700 -> 1720 us, the 256 adjoints 6420 -> 1152 (640 of them
 // the solve: 3.3 TB/s of A; floor of both halves 930).
+// Error against 80 bits on factors of N(0,1) matrices, relative to sums in 64
+// lanes and a tree (T) and to rows taken off one by one (N): T 0.93 to 1.05, N 0.55
+// to 0.91.  Two running sums over all solved rows instead of a new one for each 16:
+// 1.0 to 1.7 and 0.8 to 1.2, 60 adjoints of order 1000 655 us instead of 690.
 #include "tri_block.h"
 #include "mfma.h"
 
@@ -90,7 +94,10 @@ __device__ __forceinline__ void sweep(const T* A, long lda, int n, T* X, int ldx
       const int m = min(kb + 16 * mt + li, n - 1);
       const T* const Am = TRANS ? A + (long)m * lda : A + m;
       const T* const Xq = X + (long)min(li, NR - 1) * ldx;
-      acc_t acc2[2] = {{T(0), T(0), T(0), T(0)}, {T(0), T(0), T(0), T(0)}};  // two sums: shorter chains
+      // Every 16 products have a sum of their own, which is added to the running
+      // one: none grows with the rows already solved.
+      const acc_t zero = {T(0), T(0), T(0), T(0)};
+      acc_t acc = zero;
       for (int k0 = 16 * ks; k0 < K; k0 += 16 * G * U) {
         T a[U][4];
 #pragma unroll
@@ -106,12 +113,12 @@ __device__ __forceinline__ void sweep(const T* A, long lda, int n, T* X, int ldx
         for (int u = 0; u < U; ++u) {
           if (k0 + 16 * G * u >= K) break;
           const int kk = r0 + k0 + 16 * G * u;  // (X is zero from row n to the end of its block of 64)
+          acc_t p = zero;
 #pragma unroll
-          for (int s = 0; s < 4; ++s)
-            acc2[s & 1] = MM::op(a[u][s], Xq[TRANS ? kk + 4 * lk + s : kk + 4 * s + lk], acc2[s & 1]);
+          for (int s = 0; s < 4; ++s) p = MM::op(a[u][s], Xq[TRANS ? kk + 4 * lk + s : kk + 4 * s + lk], p);
+          acc = acc + p;
         }
       }
-      const acc_t acc = acc2[0] + acc2[1];
       if constexpr (G == 1) {
         if (li < nr) {
 #pragma unroll
