@@ -128,7 +128,8 @@ void launch_solve_err(int* err, int fail, const int* gate, hipStream_t s);
 // xchg (panel_xchg_bytes() bytes) must be zero at the start of a
 // factorization and tagbase must grow by >= 64 from one launch to the next.
 size_t panel_xchg_bytes(int max_groups);
-int panel_groups(int h);     // workgroups used at height h (0 = one workgroup, LDS only)
+int panel_groups(int h, int m);  // workgroups used at height h of an m-row matrix (0 = one, without waits)
+int panel_max_width(int h, int m, int elem);  // widest leaf there
 // mode of a leaf taller than one workgroup holds:
 enum {
   PANEL_PLAIN = 0,  // G register-resident workgroups anywhere on the device

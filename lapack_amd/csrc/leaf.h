@@ -347,8 +347,9 @@ __device__ __forceinline__ void leaf_columns(T (&v)[W], LeafLds<T, W, NTH, MULTI
   constexpr int KW = LG * VW + 2;             // words of row k
   // one workgroup's fold: LPS lanes a candidate, VPL values a lane, the
   // column searched in the candidate's last lane
-  constexpr int LPS = NW >= 8 ? 8 : 16, VPL = LPS >= LG ? 1 : LG / LPS, LV = LG / VPL;
+  constexpr int LPS = NW >= 16 ? 4 : NW >= 8 ? 8 : 16, VPL = LPS >= LG ? 1 : LG / LPS, LV = LG / VPL;
   static_assert(NW * LPS <= 64, "one lane set per wave");
+  constexpr bool LEAN = NTH >= 1024 && sizeof(T) == 8;  // (128 registers, 64 of them values)
   int tid = threadIdx.x;
   if (!PREF) asm volatile("" : "+v"(tid));  // (nothing derived from it is kept outside the leaf)
   const int lane = tid & 63;
@@ -637,13 +638,15 @@ __device__ __forceinline__ void leaf_columns(T (&v)[W], LeafLds<T, W, NTH, MULTI
           for (int c = 0; c < LG; ++c) uc[c] = lane_value(x, c);
           if (wave == NW - 1 && lane < LG) S.l[kk][lane] = x;
         } else {
-          const typename L::Msg& ms = S.wmsg[par][(lane / LPS) & (NW - 1)];
+          int ln = lane;
+          if (LEAN) asm volatile("" : "+v"(ln));  // (addresses made here, not kept over the steps)
+          const typename L::Msg& ms = S.wmsg[par][(ln / LPS) & (NW - 1)];
           // lane j of a candidate holds value (j + kk + 1) % LV of the LV
           // values around kk, and value j of the others
           const int H = kk / LV;
           T x[VPL];
 #pragma unroll
-          for (int z = 0; z < VPL; ++z) x[z] = ms.v[z * LV + ((lane + (z == H ? kk + 1 : 0)) & (LV - 1))];
+          for (int z = 0; z < VPL; ++z) x[z] = ms.v[z * LV + ((ln + (z == H ? kk + 1 : 0)) & (LV - 1))];
           const int cm = ms.meta, co = ms.org;
           const T crp = ms.rp;
           bool none;
@@ -655,9 +658,9 @@ __device__ __forceinline__ void leaf_columns(T (&v)[W], LeafLds<T, W, NTH, MULTI
 #pragma unroll
           for (int c = 0; c < LG; ++c)
             uc[c] = lane_value(x[c / LV], w0 + ((c - (c / LV == H ? kk + 1 : 0)) & (LV - 1)));
-          if (wave == NW - 1 && (lane & ~(LPS - 1)) == w0) {
+          if (wave == NW - 1 && (ln & ~(LPS - 1)) == w0) {
 #pragma unroll
-            for (int z = 0; z < VPL; ++z) S.l[kk][z * LV + ((lane + (z == H ? kk + 1 : 0)) & (LV - 1))] = x[z];
+            for (int z = 0; z < VPL; ++z) S.l[kk][z * LV + ((ln + (z == H ? kk + 1 : 0)) & (LV - 1))] = x[z];
           }
         }
         // ---- D
@@ -813,10 +816,35 @@ __device__ __forceinline__ void leaf_columns(T (&v)[W], LeafLds<T, W, NTH, MULTI
         T nl[LG], ua[LG];
 #pragma unroll
         for (int i = 0; i < LG; ++i) nl[i] = -v[i];
-        load_u(ua, 0);
+        if (!LEAN) load_u(ua, 0);
         if (MULTI) {
           // the next group's columns now; the others beside its exchanges
           apply_u(ua, nl, v + LG, k0 + LG);
+        } else if (LEAN) {
+          // (four rows of U at a time: in FP64 the products join an element one by one)
+#pragma unroll
+          for (int q = 1; q < W / LG; ++q) {
+            if (q <= rest) {
+#pragma unroll
+              for (int i0 = 0; i0 < LG; i0 += 4) {
+                T u[4], t[LG];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) u[i] = S.u[i0 + i][LG * (q - 1) + (lane & (LG - 1))];
+                T* const vq = v + LG * q;
+                if (top_wave) {
+#pragma unroll
+                  for (int c = 0; c < LG; ++c) t[c] = vq[c];
+#pragma unroll
+                  for (int i = 0; i < 4; ++i) fmac_lanes(t, u[i], nl[i0 + i]);
+#pragma unroll
+                  for (int c = 0; c < LG; ++c) vq[c] = lr >= k0 + LG ? t[c] : vq[c];
+                } else {
+#pragma unroll
+                  for (int i = 0; i < 4; ++i) fmac_lanes(vq, u[i], nl[i0 + i]);
+                }
+              }
+            }
+          }
         } else if (!PREF) {
 #pragma unroll
           for (int q = 1; q < W / LG; ++q) {

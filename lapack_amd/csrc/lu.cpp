@@ -551,7 +551,7 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
                           bool xcd0) -> int {
     const int mode = t_safe ? PANEL_TALL : xcd0 ? PANEL_XCD0 : PANEL_PLAIN;
     for (int jj = j, li = 0; jj < j + jb; ++li) {
-      const int w = std::min(leaf, j + jb - jj);
+      const int w = std::min({leaf, panel_max_width(m - jj, m, (int)sizeof(T)), j + jb - jj});
       const int rest = j + jb - jj - w;
       const RowOrg org{orgs[0], li == 0 ? nullptr : orgs[1 + ((li + 1) & 1)], orgs[1 + (li & 1)], fin_of(j),
                        rest == 0 ? 1 : 0};
@@ -580,7 +580,7 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
   };
 
   // panel 0 on the main stream
-  rc = factor_panel(0, std::min(nb, mn), s, pa, fla, xcdsplit && panel_groups(m) <= 32);
+  rc = factor_panel(0, std::min(nb, mn), s, pa, fla, xcdsplit && panel_groups(m, m) <= 32);
   for (int j = 0; j < mn && rc == 0; j += nb) {
     const int jb = std::min(nb, mn - j);
     if (j > 0) LA_TRY(hipStreamWaitEvent(s, c->ev[0], 0));  // panel j done (panel stream)
@@ -599,10 +599,10 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
     // panel (more groups) shares the GPU instead: measured at n = 32768,
     // reserving a second XCD slows the then dominant update more than it
     // speeds the panel (in FP32 as well: DSGESV 467 instead of 406 ms).
-    // The two workgroups of a panel of up to 1024 rows run on XCD 0 as well,
+    // The two workgroups of a leaf of up to 1024 rows run on XCD 0 as well,
     // but beside the update: reserving it for them takes an eighth of the GPU
     // from the update for two CUs.
-    const int pg = jbn > 0 ? panel_groups(m - jn) : 0;
+    const int pg = jbn > 0 ? panel_groups(m - jn, m) : 0;
     const bool split = xcdsplit && pg > 0 && pg <= 32;
     const int npx = split && pg > 2 ? 1 : 0;
     // While the panel holds (nearly) all of XCD 0, every launch beside it

@@ -4,9 +4,9 @@
 // The panel is A(j0:m-1, j0:j0+w-1) of the matrix being factored, held in the
 // transposed workspace T = A^T, so matrix row r of the panel is T column r and
 // its w values are contiguous.  Three forms, chosen by the panel height h:
-//   * h <= 512: one workgroup keeps the whole leaf in registers
-//     (getf2_leaf_kernel);
-//   * 512 < h <= 32768: G = h/512 workgroups keep it in registers and agree
+//   * h <= 512, and h <= 1024 in a matrix of no more rows: one workgroup keeps
+//     the whole leaf in registers (getf2_leaf_kernel) and waits for nobody;
+//   * other h <= 32768: G = h/512 workgroups keep it in registers and agree
 //     on each column's pivot through a flag-in-data exchange in device memory
 //     (the same kernel; needs its G workgroups resident together);
 //   * taller panels, and every leaf of a factorization being redone after a
@@ -55,8 +55,16 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
                                                         int* __restrict__ err, int Gp, unsigned* __restrict__ ctr,
                                                         RowOrg org) {
   constexpr int NW = NTH / 64;
-  __shared__ LeafLds<T, W, NTH, MULTI> S;
-  __shared__ int s_rank;
+  constexpr int CP = NTH >= 1024 ? 8 : 16;  // columns of a piece (below)
+  // (the leaf's first: 16 bits of offset reach the first 64 KB of LDS only)
+  __shared__ struct {
+    LeafLds<T, W, NTH, MULTI> leaf;
+    int rank;
+    T stage[NW][64][CP + 1];
+  } s_all;
+  auto& S = s_all.leaf;
+  int& s_rank = s_all.rank;
+  auto& s_stage = s_all.stage;
   const int tid = threadIdx.x;
   int G = gridDim.x;
   int b = blockIdx.x;
@@ -97,10 +105,8 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
 
   // The wave's 64 rows in and out through LDS, CP columns at a time: an access
   // of the matrix touches whole runs of CP values of 64 / CP rows (a row a lane
-  // would touch 64 lines an instruction).
-  constexpr int CP = 16;
+  // would touch 64 lines an instruction).  (16 waves' share of LDS is half.)
   constexpr int RP = 64 / CP;  // rows of one access
-  __shared__ T s_stage[NW][64][CP + 1];
   T v[W];
   {
     const int c0 = lane & (CP - 1), q0 = lane / CP;
@@ -125,7 +131,7 @@ __global__ __launch_bounds__(NTH) void getf2_leaf_kernel(T* __restrict__ Tm, lon
   // (the exchange's stores included) wherever the loop first reads v
   wait_vm();
   int my_piv, corg, zero_at;
-  leaf_columns<T, W, NTH, MULTI, XCD0, true, DIRECT>(v, S, h, w, b, G, tagbase, xbuf, err, my_piv, corg, zero_at);
+  leaf_columns<T, W, NTH, MULTI, XCD0, (NTH < 1024), DIRECT>(v, S, h, w, b, G, tagbase, xbuf, err, my_piv, corg, zero_at);
   if (lr < h) {
     const int o = j0 + (corg >= 0 && corg < h ? corg : lr);  // (out of range only after a wait gave up)
     const int po = org.pin ? org.pin[o] : o;
@@ -320,14 +326,21 @@ __global__ __launch_bounds__(256) void tall_org_kernel(int j0, int kmax, int m, 
 // Launch configurations: one workgroup with a thread a row up to 512 rows
 // (fewer threads for the shorter leaves: fewer waves to fold and to wait for).
 // Beyond that G workgroups of 512 threads; past GMAX workgroups the tall form.
+// A matrix of 513 to 1024 rows takes one workgroup of 1024 threads instead
+// (128 registers each: 32 FP64 or 64 FP32 columns), and so has no wait that could
+// give up where another kernel holds XCD 0.  Two of 512 take as long at n = 600 and
+// 800 (1.22 and 1.73 ms) and 2 % less at 1024 (2.22 ms, 2.26).  Taller matrices
+// have leaves of more than two workgroups, which wait in any case.
 static size_t tall_offset() { return (sizeof(u64) * LL_WORDS + 255) / 256 * 256; }
 // the XCD-0 panel's rank and arrival counters (zeroed with the exchange
 // buffer at the start of a factorization; each launch resets its own)
 static size_t rank_offset() { return tall_offset() + (sizeof(TallBuf) + 255) / 256 * 256; }
 size_t panel_xchg_bytes(int) { return rank_offset() + 256; }
 
-// Workgroups the panel kernel uses at height h (0 = a single workgroup).
-int panel_groups(int h) { return h <= 512 ? 0 : (h + 511) / 512; }
+// Workgroups the panel kernel uses at height h of an m-row matrix (0 = a single
+// workgroup), and the widest leaf it takes there.
+int panel_groups(int h, int m) { return h <= 512 || m <= 1024 ? 0 : (h + 511) / 512; }
+int panel_max_width(int h, int m, int elem) { return h > 512 && m <= 1024 && elem == 8 ? 32 : WMAX; }
 
 // mode: PANEL_PLAIN (G workgroups), PANEL_XCD0 (8*G blocks, those of the
 // first XCDs take part), PANEL_TALL (the form without waits).
@@ -336,15 +349,16 @@ static int launch_panel_t(T* Tm, long ldt, int j0, int w, int m, int* ipiv, int*
                           double* xchg, int* err, int mode, const RowOrg& org, hipStream_t s) {
   const int h = m - j0;
   if (h <= 0 || w <= 0) return 0;
-  if (w > WMAX) return LA_ERR_LIMIT;
+  if (w > panel_max_width(h, m, (int)sizeof(T))) return LA_ERR_LIMIT;
   u64* xb = reinterpret_cast<u64*>(xchg);
 #define LA_LEAF(W, NTH, MULTI, XCD0, DIRECT, blocks, g, ctr) \
   getf2_leaf_kernel<T, W, NTH, MULTI, XCD0, DIRECT><<<blocks, NTH, 0, s>>>(Tm, ldt, j0, w, m, ipiv, info, tagbase, xb, \
                                                                       err, g, ctr, org)
-  if (h <= 512) {
+  if (panel_groups(h, m) == 0) {
     if (h <= 128) LA_LEAF(64, 128, false, false, 0, 1, 1, nullptr);
     else if (h <= 256) LA_LEAF(64, 256, false, false, 0, 1, 1, nullptr);
-    else LA_LEAF(64, 512, false, false, 0, 1, 1, nullptr);
+    else if (h <= 512) LA_LEAF(64, 512, false, false, 0, 1, 1, nullptr);
+    else LA_LEAF((sizeof(T) == 8 ? 32 : 64), 1024, false, false, 0, 1, 1, nullptr);
     return 0;
   }
   const int G = (h + 511) / 512;
