@@ -47,6 +47,7 @@ hipStream_t ctx_stream(DevCtx* c);
 std::mutex& io_mutex(DevCtx* c);
 int io_buffer(DevCtx* c, size_t bytes, char** out);
 bool is_device_ptr(const void* p);
+bool is_pinned_ptr(const void* p);
 void phase_enable(int on);
 void phase_read(double* ms, long* calls, double* flops);
 void phase_reset();
@@ -129,12 +130,16 @@ void place(Arr<T>& a, char*& cur) {
   a.ld = std::max(a.rows, 1);
   cur += a.bytes();
 }
-// Host arrays whose columns follow each other go in one copy; with a leading
-// dimension past the rows, columns are packed through a host buffer of up to
-// PACK bytes a copy.  (A 2D copy between pageable host memory and the device
-// goes column by column: 16 us each, 8 of the 10.7 ms of a DGESV of order 500
-// on host arrays.)
-constexpr size_t PACK = (size_t)32 << 20;
+// Host arrays whose columns follow each other go in one copy.  With a leading
+// dimension past the rows:
+//   * a 2D copy from and to page-locked memory, which goes at the bus's rate for
+//     any column (57 GB/s in and out, 0.1 us a column at least), and for columns
+//     of LONG_COLUMN bytes and more;
+//   * shorter pageable columns packed through a host buffer of up to PACK bytes a
+//     copy: the 2D copy takes them one by one, 9 us in and 7 out each.  192 MB in
+//     columns of 31 / 125 / 250 / 781 KB, in + out: packed 31 / 29 / 29 / 29 ms, in
+//     2D 113 / 39 / 27 / 18 (page-locked 6.7).
+constexpr size_t PACK = (size_t)32 << 20, LONG_COLUMN = (size_t)192 << 10;
 template <class T>
 int copy_columns(Arr<T>& a, bool in, hipStream_t s) {
   if (!a.host || a.rows <= 0 || a.cols <= 0) return 0;
@@ -146,9 +151,15 @@ int copy_columns(Arr<T>& a, bool in, hipStream_t s) {
   }
   const int step = (int)std::min<size_t>((size_t)a.cols, std::max<size_t>(1, PACK / col));
   std::vector<T> buf;
-  try {
-    buf.resize((size_t)step * a.rows);
-  } catch (const std::bad_alloc&) {
+  bool packed = col < LONG_COLUMN && !is_pinned_ptr(a.user);
+  if (packed) {
+    try {
+      buf.resize((size_t)step * a.rows);
+    } catch (const std::bad_alloc&) {
+      packed = false;
+    }
+  }
+  if (!packed) {
     if (in) CK(hipMemcpy2DAsync(a.dev, col, a.user, sizeof(T) * a.user_ld, col, a.cols, hipMemcpyHostToDevice, s));
     else CK(hipMemcpy2DAsync(a.user, sizeof(T) * a.user_ld, a.dev, col, col, a.cols, hipMemcpyDeviceToHost, s));
     return 0;

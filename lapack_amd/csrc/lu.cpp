@@ -302,6 +302,12 @@ bool is_device_ptr(const void* p) {
   if (hipPointerGetAttributes(&a, p) != hipSuccess) { (void)hipGetLastError(); return false; }
   return a.type == hipMemoryTypeDevice || a.type == hipMemoryTypeManaged;
 }
+// Page-locked host memory.
+bool is_pinned_ptr(const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) { (void)hipGetLastError(); return false; }
+  return a.type == hipMemoryTypeHost;
+}
 
 // ---------------------------------------------------------- type plumbing --
 
