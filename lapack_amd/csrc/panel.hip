@@ -296,29 +296,24 @@ __global__ __launch_bounds__(256) void tall_update_kernel(T* __restrict__ Tm, lo
   if (next_keys) tall_block_max(best, brow, tb);
 }
 
-// The record of the tall form's interchanges (RowOrg), from IPIV: one
-// workgroup, thread 0 walking the at most 64 interchanges.
+// The record of the tall form's interchanges (RowOrg), from IPIV: a row a thread,
+// followed back through the at most 64 interchanges.
 __global__ __launch_bounds__(256) void tall_org_kernel(int j0, int kmax, int m, const int* __restrict__ ipiv,
                                                        RowOrg org) {
-  for (int r = j0 + (int)threadIdx.x; r < m; r += 256) org.leaf[r] = r;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = j0; k < j0 + kmax; ++k) {
-      const int p = ipiv[k] - 1;
-      if (p > k && p < m) {
-        const int t = org.leaf[k];
-        org.leaf[k] = org.leaf[p];
-        org.leaf[p] = t;
-      }
-    }
+  __shared__ int s_p[WMAX];
+  if ((int)threadIdx.x < kmax) {
+    const int k = j0 + (int)threadIdx.x, p = ipiv[k] - 1;
+    s_p[threadIdx.x] = p > k && p < m ? p : k;
   }
   __syncthreads();
-  for (int r = j0 + (int)threadIdx.x; r < m; r += 256) {
-    const int o = org.leaf[r];
-    const int po = org.pin ? org.pin[o] : o;
-    org.pout[r] = po;
-    if (org.last || r < j0 + kmax) org.fin[r] = po;
-  }
+  const int r = j0 + (int)(blockIdx.x * 256 + threadIdx.x);
+  if (r >= m) return;
+  int o = r;
+  for (int k = kmax - 1; k >= 0; --k) o = o == j0 + k ? s_p[k] : o == s_p[k] ? j0 + k : o;
+  const int po = org.pin ? org.pin[o] : o;
+  org.leaf[r] = o;
+  org.pout[r] = po;
+  if (org.last || r < j0 + kmax) org.fin[r] = po;
 }
 
 }  // namespace
@@ -377,7 +372,7 @@ static int launch_panel_t(T* Tm, long ldt, int j0, int w, int m, int* ipiv, int*
       tall_update_kernel<T><<<parts(k + 1 < kmax ? k + 1 : k), 256, 0, s>>>(Tm, ldt, j0, k, w, h, tb,
                                                                             k + 1 < kmax ? 1 : 0);
     }
-    tall_org_kernel<<<1, 256, 0, s>>>(j0, kmax, m, ipiv, org);
+    tall_org_kernel<<<(h + 255) / 256, 256, 0, s>>>(j0, kmax, m, ipiv, org);
     return 0;
   }
   unsigned* const ctr = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(xchg) + rank_offset());
