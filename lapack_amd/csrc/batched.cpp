@@ -176,12 +176,7 @@ using namespace la;
 // Persistent grids for the plan's configuration (queries the runtime once).
 static int rc_grid(lapack_amd_batch_plan* p) {
   const int nm = std::max(p->nmax, 1), b = std::max(p->batch, 1);
-  if (p->cfg == LEAF_CFG) {
-    std::vector<int> sorted = p->n;
-    std::sort(sorted.begin(), sorted.end(), std::greater<int>());
-    if (p->elem == 8) batched_leaf_plan<double>(p->batch, sorted.data(), &p->leaf);
-    else batched_leaf_plan<float>(p->batch, sorted.data(), &p->leaf);
-  } else {
+  if (p->cfg != LEAF_CFG) {
     const int gf = p->elem == 8 ? batched_getrf_grid<double>(p->cfg, b, nm) : batched_getrf_grid<float>(p->cfg, b, nm);
     if (gf < 0) return gf;
     p->grid_f = gf;
@@ -231,6 +226,12 @@ int lapack_amd_batch_plan_create(lapack_amd_batch_plan** out, int batch, const i
   }
   p->cfg = default_cfg(std::max(p->nmax, 1), p->elem);
   if (p->cfg < 0) { lapack_amd_batch_plan_destroy(p); return LA_ERR_LIMIT; }
+  if (p->nmax <= batched_leaf_nmax()) {  // (here, so that set_config allocates nothing)
+    std::vector<int> sorted(batch);
+    for (int i = 0; i < batch; ++i) sorted[i] = p->n[order[i]];
+    if (dbl) batched_leaf_plan<double>(batch, sorted.data(), &p->leaf);
+    else batched_leaf_plan<float>(batch, sorted.data(), &p->leaf);
+  }
   if (autotune && batch > 0 && p->cfg != LEAF_CFG) {
     long long sum = 0;
     for (int v : p->n) sum += v;

@@ -276,3 +276,61 @@ def test_dsgesv_reports_wait_failure(dev):
     aa = np.array(a, order="F")
     info, it = la.dsgesv(n, 1, aa, n, ipiv, b, n, x, n)
     assert info == 0 and it > 0
+
+
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("n,nrhs", [(300, 1), (512, 1), (513, 1), (1500, 1), (300, 3), (700, 17)])
+def test_getrs_wait_failure_every_form(dev, trans, n, nrhs):
+    """As test_getrs_wait_failure for one right-hand side, whose sweeps, small
+    permutations and report are their own, and for a slice of one column over."""
+    import torch
+    a, b = la.matrix(2, 1601, n, n), la.matrix(2, 1602, n, nrhs)
+    lu, p, info = gpu_getrf(a)
+    assert info == 0
+    d_lu, d_p, d_b = to_dev(lu), to_dev(p.reshape(-1, 1).astype(np.int32)), to_dev(b)
+    la.device_status(clear=True)
+    la.test_fail_waits(1)
+    assert la.dgetrs_async(trans, n, nrhs, d_lu, n, d_p, d_b, n) == 0
+    torch.cuda.synchronize()
+    assert np.array_equal(from_dev(d_b, (n, nrhs)).view(np.int64), b.view(np.int64))
+    assert la.device_status(clear=True) & 1
+    assert la.dgetrs_async(trans, n, nrhs, d_lu, n, d_p, d_b, n) == 0  # the next one solves
+    torch.cuda.synchronize()
+    assert oracle.dget02(a, from_dev(d_b, (n, nrhs)), b, trans) < THRESH
+    assert la.device_status(clear=True) == 0
+    la.test_fail_waits(1)
+    bb = np.array(b, order="F")
+    assert la.dgetrs(trans, n, nrhs, d_lu, n, d_p, bb, n) == 0
+    assert oracle.dget02(a, bb, b, trans) < THRESH
+    la.device_status(clear=True)
+
+
+@pytest.mark.parametrize("waits", [1, 2])
+@pytest.mark.parametrize("n,nrhs", [(300, 1), (700, 1), (700, 3)])
+def test_gesv_wait_failure_recovers(dev, n, nrhs, waits):
+    """DGESV's solve is enqueued behind the factorization: where the first gives up,
+    or both, the call redoes them and returns the reference's result."""
+    a, b = la.matrix(2, 1701, n, n), la.matrix(2, 1702, n, nrhs)
+    aa, bb, p = np.array(a, order="F"), np.array(b, order="F"), np.zeros(n, np.int32)
+    la.device_status(clear=True)
+    la.test_fail_waits(waits)
+    assert la.dgesv(n, nrhs, aa, n, p, bb, n) == 0
+    la.test_fail_waits(0)
+    assert la.device_status(clear=True) & 1
+    assert np.array_equal(p, oracle.dgetrf(a)[1])
+    assert oracle.dget02(a, bb, b) < THRESH
+
+
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("n,nrhs", [(300, 17), (300, 33), (129, 18), (200, 32)])
+def test_slices_of_sixteen_right_hand_sides(dev, trans, n, nrhs):
+    """Past 16 right-hand sides the sweeps take slices, the last of one, a few or 16 columns."""
+    a, b = la.matrix(2, 1801 + n, n, n), la.matrix(2, 1802, n, nrhs)
+    lu, p, _ = oracle.dgetrf(a)
+    d_b = to_dev(b)
+    assert la.dgetrs(trans, n, nrhs, to_dev(lu), n, to_dev(p.reshape(-1, 1).astype(np.int32)), d_b, n) == 0
+    x = from_dev(d_b, (n, nrhs))
+    ref = oracle.dgetrs(lu, p, np.asfortranarray(b), trans)[0]
+    assert oracle.dget02(a, x, b, trans) < THRESH
+    cond = np.linalg.cond(a)
+    assert np.abs(x - ref).max() <= 4 * n * EPS * cond * np.abs(ref).max()  # (each within 2 n eps cond)
