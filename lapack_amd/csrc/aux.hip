@@ -470,18 +470,10 @@ __global__ __launch_bounds__(256) void trtri_kernel(int n, int nb, const T* __re
 // ---- copies and fills -----------------------------------------------------
 template <class T>
 __global__ __launch_bounds__(256) void copy_kernel(int rows, int cols, const T* __restrict__ src, long lds,
-                                                   T* __restrict__ dst, long ldd, int nskip,
-                                                   const int* __restrict__ skip) {
+                                                   T* __restrict__ dst, long ldd, const int* __restrict__ skip) {
   if (skip && *skip) return;
-  // nskip: blocks dispatched to XCDs 0 .. nskip-1 (blockIdx % 8) leave at once
-  long lb = blockIdx.x, ng = gridDim.x;
-  if (nskip) {
-    if ((int)(blockIdx.x % 8) < nskip) return;
-    lb = (long)(blockIdx.x / 8) * (8 - nskip) + (blockIdx.x % 8 - nskip);
-    ng = (long)(gridDim.x / 8) * (8 - nskip);
-  }
   const long tot = (long)rows * cols;
-  for (long e = lb * 256 + threadIdx.x; e < tot; e += ng * 256) {
+  for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < tot; e += (long)gridDim.x * 256) {
     const long i = e % rows, j = e / rows;
     dst[i + j * ldd] = src[i + j * lds];
   }
@@ -644,21 +636,15 @@ void launch_trtri_blocks_s(bool upper, bool unit, int n, int nb, const float* U,
                            long ldw, hipStream_t s) {
   launch_trtri_t<float>(upper, unit, n, nb, U, ldu, W, ldw, s);
 }
-static int copy_grid(long work, int nskip) {
-  const int g = grid_for(work);
-  return nskip ? (g + (8 - nskip) - 1) / (8 - nskip) * 8 : g;
-}
 void launch_copy_d(int rows, int cols, const double* src, long lds, double* dst, long ldd, hipStream_t s,
-                   int nskip, const int* skip) {
+                   const int* skip) {
   if (rows > 0 && cols > 0)
-    copy_kernel<double><<<copy_grid((long)rows * cols, nskip), 256, 0, s>>>(rows, cols, src, lds, dst, ldd, nskip,
-                                                                            skip);
+    copy_kernel<double><<<grid_for((long)rows * cols), 256, 0, s>>>(rows, cols, src, lds, dst, ldd, skip);
 }
 void launch_copy_s(int rows, int cols, const float* src, long lds, float* dst, long ldd, hipStream_t s,
-                   int nskip, const int* skip) {
+                   const int* skip) {
   if (rows > 0 && cols > 0)
-    copy_kernel<float><<<copy_grid((long)rows * cols, nskip), 256, 0, s>>>(rows, cols, src, lds, dst, ldd, nskip,
-                                                                           skip);
+    copy_kernel<float><<<grid_for((long)rows * cols), 256, 0, s>>>(rows, cols, src, lds, dst, ldd, skip);
 }
 void launch_fill_u32(unsigned* p, size_t n, unsigned v, hipStream_t s) {
   if (n) fill_kernel<unsigned><<<grid_for((long)n), 256, 0, s>>>(p, n, v);

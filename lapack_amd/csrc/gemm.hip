@@ -20,7 +20,7 @@
 // Workgroups are mapped XCD-aware: blockIdx % 8 selects the XCD (round-robin
 // dispatch), and each XCD receives a contiguous, M-grouped range of tiles so
 // the A row panels and B column panels it touches stay in its own L2.
-#include "la_common.h"
+#include "mfma.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -32,26 +32,7 @@ constexpr int BM = 128, BN = 128, BK = 16, NT = 256;
 constexpr int GROUP_M = 8;
 constexpr int NXCD = 8;
 
-template <class T> struct Mfma;
-template <> struct Mfma<double> {
-  typedef la_d4 acc_t;
-  static __device__ __forceinline__ acc_t op(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  // Accumulator register r of lane l holds D[l/16 + 4r][l%16] (measured on
-  // gfx950; the f32 form below differs).
-  static __device__ __forceinline__ int row(int lk, int r) { return lk + 4 * r; }
-  static constexpr int APAD = 8;  // (BM+APAD)*8 bytes = 64 mod 128
-};
-template <> struct Mfma<float> {
-  typedef la_f4 acc_t;
-  static __device__ __forceinline__ acc_t op(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  // Accumulator register r of lane l holds D[4*(l/16) + r][l%16].
-  static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
-  static constexpr int APAD = 16;
-};
+template <class T> constexpr int APAD = sizeof(T) == 8 ? 8 : 16;  // FP64: (BM+APAD)*8 bytes = 64 mod 128
 
 // Products are issued as C^T = B^T A^T (the B fragment in the MFMA's A
 // slot), so block (i, j) of a wave's 64x64 C tile holds, in register r of
@@ -108,7 +89,7 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(int M, int N, int K, T alph
                                                      T* __restrict__ C, long ldc, int tm, int tn,
                                                      int chunk, int nxcd) {
   typedef typename Mfma<T>::acc_t acc_t;
-  constexpr int AST = BM + Mfma<T>::APAD;  // As row stride
+  constexpr int AST = BM + APAD<T>;  // As row stride
   constexpr int BST = BK + 1;              // Bs row stride
   __shared__ T As[2][BK * AST];
   __shared__ T Bs[2][BN * BST];
@@ -263,7 +244,7 @@ __global__ __launch_bounds__(WM * WN * 64) void update_big_kernel(int M, int N, 
   typedef typename Mfma<T>::acc_t acc_t;
   constexpr int NTB = WM * WN * 64;
   constexpr int TBM = WM * 64, TBN = WN * 64;
-  constexpr int AST = TBM + Mfma<T>::APAD;
+  constexpr int AST = TBM + APAD<T>;
   constexpr int BST = BK + 1;
   constexpr int LA = TBM * BK / NTB, LB = TBN * BK / NTB;
   __shared__ T As[2][BK * AST];
@@ -620,7 +601,7 @@ __global__ __launch_bounds__(512) void update_pipe_kernel(int K, const T* __rest
                                                          long ldc, int tm, int tn, int chunk, int nxcd) {
   typedef typename Mfma<T>::acc_t acc_t;
   constexpr int NTB = 512, TBM = 128, TBN = 128, PBK = 32;
-  constexpr int AST = TBM + Mfma<T>::APAD;
+  constexpr int AST = TBM + APAD<T>;
   constexpr int BST = PBK + 1;
   constexpr int LA = TBM * PBK / NTB, LB = TBN * PBK / NTB;
   constexpr int NG = 8;  // accumulator blocks per wave = C read groups per tile
@@ -803,7 +784,7 @@ __global__ __launch_bounds__(256) void gemm64_kernel(int M, int N, int K, T alph
   }
   typedef typename Mfma<T>::acc_t acc_t;
   constexpr int TS = 64;
-  constexpr int AST = TS + Mfma<T>::APAD;
+  constexpr int AST = TS + APAD<T>;
   constexpr int BST = BK + 1;
   __shared__ T As[2][BK * AST];
   __shared__ T Bs[2][TS * BST];
@@ -898,13 +879,13 @@ void launch_update_t(int m, int n, int k, const T* A, long lda, const T* B, long
 
 template <class T>
 void launch_gemm_t(char ta, char tb, int m, int n, int k, T alpha, const T* A, long lda, const T* B,
-                   long ldb, T beta, T* C, long ldc, hipStream_t s, int nskip) {
+                   long ldb, T beta, T* C, long ldc, hipStream_t s) {
   if (m <= 0 || n <= 0) return;
   // BLAS quick return (BLAS/SRC/dgemm.f:298-299).
   if ((alpha == T(0) || k <= 0) && beta == T(1)) return;
   const int tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;
   const int tiles = tm * tn;
-  const int nx = NXCD - nskip;
+  const int nx = NXCD;
   const int chunk = (tiles + nx - 1) / nx;
   const dim3 grid(chunk * NXCD);
   const bool TA = (ta == 'T' || ta == 't' || ta == 'C' || ta == 'c');
@@ -912,11 +893,11 @@ void launch_gemm_t(char ta, char tb, int m, int n, int k, T alpha, const T* A, l
   if (k <= 0 || alpha == T(0)) k = 0;  // C <- beta*C (dgemm.f:303-318)
   // C - A*B, the trailing-update form: the update kernels (C read into the
   // accumulators first, A negated)
-  if (!TA && !TB && nskip == 0 && k > 0 && alpha == T(-1) && beta == T(1)) {
+  if (!TA && !TB && k > 0 && alpha == T(-1) && beta == T(1)) {
     launch_update_t<T>(m, n, k, A, lda, B, ldb, C, ldc, 0, s, true);
     return;
   }
-  if (!TA && !TB && nskip == 0 && tiles < 64 && k >= 64) {
+  if (!TA && !TB && tiles < 64 && k >= 64) {
     const int tm64 = (m + 63) / 64, tn64 = (n + 63) / 64;
     gemm64_kernel<T><<<dim3(tm64 * tn64), 256, 0, s>>>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tm64);
     return;
@@ -1118,8 +1099,8 @@ void launch_update_t(int m, int n, int k, const T* A, long lda, const T* B, long
 }  // namespace
 
 void launch_dgemm(char ta, char tb, int m, int n, int k, double alpha, const double* A, long lda,
-                  const double* B, long ldb, double beta, double* C, long ldc, hipStream_t s, int nskip) {
-  launch_gemm_t<double>(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s, nskip);
+                  const double* B, long ldb, double beta, double* C, long ldc, hipStream_t s) {
+  launch_gemm_t<double>(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s);
 }
 void launch_dgemm_update(int m, int n, int k, const double* A, long lda, const double* B, long ldb, double* C,
                          long ldc, int nskip, hipStream_t s) {
@@ -1130,8 +1111,8 @@ void launch_sgemm_update(int m, int n, int k, const float* A, long lda, const fl
   launch_update_t<float>(m, n, k, A, lda, B, ldb, C, ldc, nskip, s);
 }
 void launch_sgemm(char ta, char tb, int m, int n, int k, float alpha, const float* A, long lda,
-                  const float* B, long ldb, float beta, float* C, long ldc, hipStream_t s, int nskip) {
-  launch_gemm_t<float>(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s, nskip);
+                  const float* B, long ldb, float beta, float* C, long ldc, hipStream_t s) {
+  launch_gemm_t<float>(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s);
 }
 
 }  // namespace la

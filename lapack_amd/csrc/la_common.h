@@ -36,9 +36,10 @@ __device__ __forceinline__ void wait_vm() { __builtin_amdgcn_s_waitcnt(0x0F70); 
 
 // C <- alpha*op(A)*op(B) + beta*C, column-major, FP64 MFMA.
 void launch_dgemm(char ta, char tb, int m, int n, int k, double alpha, const double* A, long lda,
-                  const double* B, long ldb, double beta, double* C, long ldc, hipStream_t s, int nskip = 0);
+                  const double* B, long ldb, double beta, double* C, long ldc, hipStream_t s);
 // The DGETRF trailing update C <- C - A*B (its own kernel symbols).
-// nskip: leave XCDs 0 .. nskip-1 to a concurrent panel kernel.
+// nskip (updates and swap_trsm): no work on XCDs 0 .. nskip-1, which a
+// concurrent panel keeps for itself.
 void launch_dgemm_update(int m, int n, int k, const double* A, long lda, const double* B, long ldb, double* C,
                          long ldc, int nskip, hipStream_t s);
 // FP32 update with operands rounded to FP16 (kind 1) or BF16 (kind 2), FP32
@@ -49,7 +50,7 @@ void launch_sgemm_update(int m, int n, int k, const float* A, long lda, const fl
                          int nskip, hipStream_t s);
 // Same in FP32 (MFMA f32).
 void launch_sgemm(char ta, char tb, int m, int n, int k, float alpha, const float* A, long lda,
-                  const float* B, long ldb, float beta, float* C, long ldc, hipStream_t s, int nskip = 0);
+                  const float* B, long ldb, float beta, float* C, long ldc, hipStream_t s);
 
 // out(j,i) = in(i,j): in is rows x cols with ld_in, out cols x rows with ld_out.
 // skip (optional device int): nothing is written when *skip != 0.
@@ -105,13 +106,11 @@ void launch_trtri_blocks_d(bool upper, bool unit, int n, int nb, const double* U
 void launch_trtri_blocks_s(bool upper, bool unit, int n, int nb, const float* U, long ldu, float* W,
                            long ldw, hipStream_t s);
 // Copy a rows x cols column-major block.
-// nskip (copy, interchanges, GEMM, update): no work on XCDs 0 .. nskip-1,
-// which a concurrent panel keeps for itself.
 // skip (optional device int): nothing is written when *skip != 0.
 void launch_copy_d(int rows, int cols, const double* src, long lds, double* dst, long ldd, hipStream_t s,
-                   int nskip = 0, const int* skip = nullptr);
+                   const int* skip = nullptr);
 void launch_copy_s(int rows, int cols, const float* src, long lds, float* dst, long ldd, hipStream_t s,
-                   int nskip = 0, const int* skip = nullptr);
+                   const int* skip = nullptr);
 void launch_fill_u32(unsigned* p, size_t n, unsigned v, hipStream_t s);
 void launch_fill_i32(int* p, size_t n, int v, hipStream_t s);
 // x[i] uniform in [-1, 1) from a counter-based hash of (seed, i)
@@ -133,7 +132,7 @@ int panel_max_width(int h, int m, int elem);  // widest leaf there
 // mode of a leaf taller than one workgroup holds:
 enum {
   PANEL_PLAIN = 0,  // G register-resident workgroups anywhere on the device
-  PANEL_XCD0 = 1,   // the same on XCD 0 only (8*G blocks launched, every eighth takes part)
+  PANEL_XCD0 = 1,   // the same on XCD 0 only (8*G blocks launched, those that run there take part)
   PANEL_TALL = 2,   // column by column over HBM, no workgroup waits for another
 };
 int launch_getf2_panel_d(double* T, long ldt, int j0, int w, int m, int* ipiv, int* info, unsigned tagbase,

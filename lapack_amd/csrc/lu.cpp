@@ -52,7 +52,7 @@ struct DevCtx {
   bool ws_used = false;
   hipStream_t pstream = nullptr;      // panel stream (look-ahead)
   hipStream_t ustream = nullptr;      // trailing-update stream
-  hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   char* mp = nullptr;            // buffers of the mixed-precision solvers
   size_t mp_bytes = 0;
   int* status = nullptr;         // sticky device word: bit 0 = a bounded wait gave up
@@ -314,8 +314,8 @@ bool is_pinned_ptr(const void* p) {
 template <class T> struct K;
 template <> struct K<double> {
   static void gemm(char ta, char tb, int m, int n, int k, double al, const double* A, long lda, const double* B,
-                   long ldb, double be, double* C, long ldc, hipStream_t s, int nskip = 0) {
-    launch_dgemm(ta, tb, m, n, k, al, A, lda, B, ldb, be, C, ldc, s, nskip);
+                   long ldb, double be, double* C, long ldc, hipStream_t s) {
+    launch_dgemm(ta, tb, m, n, k, al, A, lda, B, ldb, be, C, ldc, s);
   }
   static void update(int m, int n, int k, const double* A, long lda, const double* B, long ldb, double* C, long ldc,
                      int nskip, hipStream_t s) {
@@ -340,9 +340,9 @@ template <> struct K<double> {
                            hipStream_t s) {
     launch_trtri_blocks_d(up, unit, n, nb, U, ldu, W, ldw, s);
   }
-  static void copy(int r, int c, const double* src, long ls, double* dst, long ld, hipStream_t s, int nskip = 0,
+  static void copy(int r, int c, const double* src, long ls, double* dst, long ld, hipStream_t s,
                    const int* skip = nullptr) {
-    launch_copy_d(r, c, src, ls, dst, ld, s, nskip, skip);
+    launch_copy_d(r, c, src, ls, dst, ld, s, skip);
   }
   static int panel(double* T, long ldt, int j0, int w, int m, int* ipiv, int* info, unsigned tagbase, double* x,
                    int* err, int mode, const RowOrg& org, hipStream_t s) {
@@ -356,8 +356,8 @@ static thread_local int t_upd_kind = 0;
 
 template <> struct K<float> {
   static void gemm(char ta, char tb, int m, int n, int k, float al, const float* A, long lda, const float* B,
-                   long ldb, float be, float* C, long ldc, hipStream_t s, int nskip = 0) {
-    launch_sgemm(ta, tb, m, n, k, al, A, lda, B, ldb, be, C, ldc, s, nskip);
+                   long ldb, float be, float* C, long ldc, hipStream_t s) {
+    launch_sgemm(ta, tb, m, n, k, al, A, lda, B, ldb, be, C, ldc, s);
   }
   static void update(int m, int n, int k, const float* A, long lda, const float* B, long ldb, float* C, long ldc,
                      int nskip, hipStream_t s) {
@@ -385,9 +385,9 @@ template <> struct K<float> {
                            hipStream_t s) {
     launch_trtri_blocks_s(up, unit, n, nb, U, ldu, W, ldw, s);
   }
-  static void copy(int r, int c, const float* src, long ls, float* dst, long ld, hipStream_t s, int nskip = 0,
+  static void copy(int r, int c, const float* src, long ls, float* dst, long ld, hipStream_t s,
                    const int* skip = nullptr) {
-    launch_copy_s(r, c, src, ls, dst, ld, s, nskip, skip);
+    launch_copy_s(r, c, src, ls, dst, ld, s, skip);
   }
   static int panel(float* T, long ldt, int j0, int w, int m, int* ipiv, int* info, unsigned tagbase, double* x,
                    int* err, int mode, const RowOrg& org, hipStream_t s) {
@@ -501,7 +501,7 @@ int getrf_device(int m, int n, T* A, long lda, int* ipiv, int* info, hipStream_t
     // streams of their own, fenced to the caller's stream
     LA_TRY(hipStreamCreateWithFlags(&c->pstream, hipStreamNonBlocking));
     LA_TRY(hipStreamCreateWithFlags(&c->ustream, hipStreamNonBlocking));
-    for (int i = 0; i < 5; ++i) LA_TRY(hipEventCreateWithFlags(&c->ev[i], hipEventDisableTiming));
+    for (int i = 0; i < 4; ++i) LA_TRY(hipEventCreateWithFlags(&c->ev[i], hipEventDisableTiming));
   }
   hipStream_t sp = c->pstream;
   hipStream_t s_user = s;
@@ -728,7 +728,7 @@ void getrs_chain(char trans, int n, int nrhs, const T* A, long lda, const int* i
     K<T>::gather(n, nrhs, perm, B, ldb, X, ldx, s);                         // X = P*B (dgetrs.f:187)
     launch_tri_chain<T>(0, n, nrhs, A, lda, X, ldx, Y, ldx, ctl, cerr, s);  // L Y = X (dgetrs.f:191)
     launch_tri_chain<T>(1, n, nrhs, A, lda, Y, ldx, X, ldx, ctl, cerr, s);  // U X = Y (dgetrs.f:197)
-    K<T>::copy(n, nrhs, X, ldx, B, ldb, s, 0, cerr);
+    K<T>::copy(n, nrhs, X, ldx, B, ldb, s, cerr);
   } else {
     K<T>::copy(n, nrhs, B, ldb, X, ldx, s);
     launch_tri_chain<T>(2, n, nrhs, A, lda, X, ldx, Y, ldx, ctl, cerr, s);  // U^T Y = B (dgetrs.f:205)

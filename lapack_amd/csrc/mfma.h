@@ -1,6 +1,6 @@
 // mfma.h -- the 16 x 16 x 4 matrix-core product in FP64 and FP32: lane l holds
 // A(l % 16, l / 16) and B(l / 16, l % 16) of a step; accumulator register r of
-// lane l holds D(row(l / 16, r), l % 16).
+// lane l holds D(row(l / 16, r), l % 16) (measured; the two precisions differ).
 #pragma once
 #include "la_common.h"
 

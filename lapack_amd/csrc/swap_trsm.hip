@@ -25,25 +25,10 @@
 // dependent steps), by the matrix cores and the triangle's re-reads from L2
 // for all columns of a large matrix.
 #include "leaf.h"
+#include "mfma.h"
 
 namespace la {
 namespace {
-
-template <class T> struct SMfma;
-template <> struct SMfma<double> {
-  typedef la_d4 acc_t;
-  static __device__ __forceinline__ acc_t op(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return lk + 4 * r; }
-};
-template <> struct SMfma<float> {
-  typedef la_f4 acc_t;
-  static __device__ __forceinline__ acc_t op(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
-};
 
 constexpr int SB = 64;        // rows of a solve block
 constexpr int SC = 16;        // columns of A a workgroup owns
@@ -77,7 +62,7 @@ __global__ __launch_bounds__(SNT) void swap_trsm_kernel(T* __restrict__ Tm, long
                                                         int c1, int s0, int s1, const int* __restrict__ ipiv,
                                                         const int* __restrict__ org, int nsolve, int nblk,
                                                         int nskip) {
-  typedef SMfma<T> MM;
+  typedef Mfma<T> MM;
   typedef typename MM::acc_t acc_t;
   constexpr int NW = SNT / 64;
   constexpr int RPP = SNT / SC;          // rows a pass moves
