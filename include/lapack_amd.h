@@ -233,8 +233,9 @@ int lapack_amd_dgesv_adjoint_async(int n, int nrhs, const double* d_lu, int lda,
  * -- for orders past 512, with autotune != 0 -- times the kernel
  * configurations (panel width NB, workgroup size) on synthetic matrices of the
  * plan's sizes and keeps the fastest; up to 512 it takes the configuration
- * (32, 512), which needs no trial.  Creating a plan allocates; the *_batched_async launches do
- * not, and may be captured in a hipGraph and replayed. */
+ * (32, 512), which needs no trial (the plan's tuned_ms is then 0).  Creating a
+ * plan allocates; the *_batched_async launches do not, and may be captured in
+ * a hipGraph and replayed. */
 typedef struct lapack_amd_batch_plan lapack_amd_batch_plan;
 int lapack_amd_batch_plan_create(lapack_amd_batch_plan** plan, int batch, const int* n, char precision,
                                  int autotune);
@@ -385,7 +386,8 @@ const char* lapack_amd_version(void);
 
 /* The multi-workgroup panel kernels of DGETRF/SGETRF and the triangular
  * sweeps of DGETRS/SGETRS wait for each other's workgroups with bounded
- * waits.  When a wait gives up (its workgroups were not all resident, e.g.
+ * waits.  (Matrices of up to 1024 rows are factored without any.)  When a wait
+ * gives up (its workgroups were not all resident, e.g.
  * another process held the CUs), every kernel still runs to its end and:
  *   - getrf leaves A exactly as passed and writes INFO = LA_ERR_SYNC;
  *   - getrs leaves B exactly as passed;

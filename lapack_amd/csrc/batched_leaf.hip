@@ -29,7 +29,8 @@
 // matrix in FP64) where the batch exceeds the caches.  10000 matrices of
 // order 16..512: 28.2 ms (best panel form 62.9); the substitution keeps 8 steps'
 // coefficients at a time and its rounds are not unrolled (32.6 ms with all of
-// them in flight: the registers then spilled).
+// them in flight, which spilled far more than the 25 registers that the FP64 forms
+// of 256 and 512 threads still do, 104 and 108 bytes of scratch a lane).
 #include "leaf.h"
 #include "mfma.h"
 

@@ -768,12 +768,12 @@ __global__ __launch_bounds__(512) void update_pipe_kernel(int K, const T* __rest
 }
 
 // Small products (C = alpha*A*B + beta*C, A and B untransposed, few 128x128
-// tiles: the DTRSM product of the next panel's 256 columns is 256x256x256,
-// four such tiles): 64x64 tiles, so that 16 workgroups share the work.  A
+// tiles: a 256x256x256 product is four of them): 64x64 tiles, so that 16
+// workgroups share the work.  A
 // 256-thread workgroup = 2x2 waves of 2x2 MFMA blocks, BK = 16, double-
 // buffered LDS, products issued as C^T = B^T A^T as in gemm_kernel.
 // UPD: the trailing-update instance (alpha = -1, beta = 1), a symbol of its
-// own so that traces and counters tell it from the DTRSM products.
+// own so that traces and counters tell it from the other products.
 template <class T, bool UPD = false>
 __global__ __launch_bounds__(256) void gemm64_kernel(int M, int N, int K, T alpha, const T* __restrict__ A,
                                                      long lda, const T* __restrict__ B, long ldb, T beta,

@@ -12,9 +12,9 @@
 //     i.e. for workgroups already running, so every wait ends;
 //   * thread (i, g) owns row i of the block and the columns c in
 //     [16g, 16g+16) of every 64-column tile of M it depends on; tiles are
-//     read straight from HBM, up to two dependency blocks per round: their
-//     flags are polled together, their x blocks staged in LDS together, and
-//     the round's products are summed on their own before they join the
+//     read straight from HBM, up to two dependency blocks per round: a value
+//     of each x block is polled together, the blocks staged in LDS together,
+//     and the round's products are summed on their own before they join the
 //     running sum (two-level summation: no sum runs over more than 64 terms
 //     of one round or one term per round).  The block's last dependency --
 //     the one finished most recently -- gets a round of its own, so the
@@ -25,8 +25,9 @@
 //     not a 64-step chain;
 //   * the four partial sums per row are added in LDS, y = b + acc, and
 //     x = inv(M_dd) y, one wavefront per four right-hand sides;
-//   * x is stored with device-coherent stores, the stores are waited for,
-//     and the block's flag is raised.
+//   * x is stored with device-coherent stores.  Its place held a sentinel, a
+//     NaN with a payload of its own (tri_block.h), so that every value tells by
+//     itself whether it is there: no flag, and no wait for the stores.
 // Every wait is bounded; one that gives up sets *err, and the other waits
 // poll *err and give up as well, so every workgroup runs to its end (the
 // caller then leaves B as it was and reports the failure).

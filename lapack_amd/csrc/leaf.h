@@ -95,8 +95,11 @@ __device__ __forceinline__ unsigned wave_max_recip(unsigned hi, float x, float* 
   return lanes_max<1, 64>(hi);
 }
 __device__ __forceinline__ unsigned wave_max_recip(unsigned hi, double x, double* rp) {
-  // the correctly rounded division's own sequence (scaled operands, reciprocal
-  // refined twice, quotient, its residual, fix-up), in the DPP wait states
+  // 1 / x as the CDNA instruction set documents its division instructions:
+  // operands scaled (v_div_scale), the estimate v_rcp refined by two Newton steps,
+  // the quotient corrected by its residual (Markstein, IBM J. R&D 34, 1990), the
+  // scaling undone and special operands fixed up (v_div_fmas, v_div_fixup); laid
+  // out in the DPP wait states
 #define LA_STEP __builtin_amdgcn_sched_barrier(0)
   bool f0, f1;
   unsigned v = hi;
@@ -215,8 +218,8 @@ __device__ __forceinline__ bool recip_ok(T piv) {
 // rows of a group before every workgroup has read those of the group before
 // (each reads them before it publishes its next candidate), so one buffer
 // suffices for the rows.  The exchange buffer must be zero before the first
-// launch of a factorization (flags only grow after that: tagbase advances by
-// 64 per launch).
+// launch of a factorization; after that flags only grow (tagbase advances by 64
+// per launch), so a word of an earlier leaf never passes for a current one.
 constexpr int LG = 8;                        // columns of a group
 constexpr int MSGS = 32;                     // words of a candidate's slot (padded)
 constexpr size_t MSG_PAR = 2880;             // candidates of one column + row k
@@ -236,8 +239,11 @@ __device__ __forceinline__ u64 ll_word(unsigned payload, unsigned flag) {
 // (about 1000 of 5450 cycles a column) and takes the reciprocal out of the chain;
 // a round of loads is what the polls take more as the waves grow (DGETRF at n =
 // 1024 / 4096 / 8192: 2.30 / 10.86 / 24.04 -> 2.18 / 10.04 / 23.04 ms, SGETRF 2.03 /
-// 9.58 / 20.52 -> 1.88 / 8.46 / 18.56).  A flag's top bit tells these upper words from the other ones (whose
-// flags stay below 2^31).
+// 9.58 / 20.52 -> 1.88 / 8.46 / 18.56).  A flag's top bit tells these upper words from
+// the other ones (whose flags stay below 2^31); the 19 bits of the flag beside it
+// repeat after 8192 leaves, which no factorization has that uses them (up to 8192
+// rows; even leaves of one column are no more), and between factorizations the
+// buffer is zeroed.
 constexpr int DIRECT_CANDS = 128;
 constexpr int DIRECT_ROWK = 2 * DIRECT_CANDS;     // row k's words
 constexpr int DIRECT_VALUES = DIRECT_ROWK + 32;   // the candidates' values

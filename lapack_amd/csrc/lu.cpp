@@ -57,9 +57,9 @@ struct DevCtx {
   size_t mp_bytes = 0;
   int* status = nullptr;         // sticky device word: bit 0 = a bounded wait gave up
   bool xcd8 = false;             // 8 XCDs of >= 32 CUs: the panel may own XCD 0
-  // flag base of the next panel launch: grows by 64 per launch across calls,
-  // so that an exchange word left from an earlier launch (in memory or in an
-  // XCD's L2) never carries a current flag
+  // flag base of the next panel launch: grows by 64 per launch across calls.
+  // Within a factorization no two launches share a flag; words of an earlier
+  // one are gone, as every factorization zeroes the exchange buffer.
   unsigned leaf_tag = 0;
   std::mutex mu;     // guards ws and the launch sequence of one call
   std::mutex io_mu;  // guards io across a whole synchronous call
@@ -121,7 +121,7 @@ int tune_nb_for(int n) {
   if (v <= 0) v = env_int("LAPACK_AMD_NB", 0);
   if (v <= 0 && n > 0) v = table_entry(n).nb;
   if (v <= 0) v = 256;
-  return std::max(1, std::min(v, 256));  // the triangle-inverse kernel covers <= 256
+  return std::max(1, std::min(v, 256));  // the widest block of swap_trsm.hip
 }
 int tune_leaf_for(int n) {
   if (t_force_leaf > 0) return t_force_leaf;

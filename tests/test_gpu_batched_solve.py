@@ -1,6 +1,6 @@
 """The batch's triangular solves (SRC/dgetrs.f:181-218) at the edges of their
 blocks of 64 rows, sub-blocks of 16 and passes of 4 or 8 right-hand sides, in
-each of the three workgroup sizes, against the oracle's DGETRS on the same
+each of the two workgroup sizes, against the oracle's DGETRS on the same
 factors.
 
 Tolerance: the matrices are random rows plus 4 sqrt(n) on the diagonal, their
