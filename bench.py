@@ -395,14 +395,14 @@ def batch_workload(precision, seed=4):
     f_s = sum(2.0 * n * n * r for n, r in zip(ns, nrhs))
     byt = sum(2.0 * es * n * n for n in ns)
     peak = PEAK_FP64 if precision == "d" else PEAK_FP32
-    nb, nt, _ = plan.config()
+    nb, nt, trial_ms = plan.config()
     out = {"workload": f"10000 uneven systems ({'FP64' if precision == 'd' else 'FP32'}), n in [16,512], nrhs in [1,4]",
            "getrf_ms": round(t_f, 3), "getrs_ms": round(t_s, 3),
            "tflops": round((f_f + f_s) / (t_f + t_s) / 1e9, 3),
            "getrf_tflops": round(f_f / t_f / 1e9, 3),
            "frac_peak": round(f_f / t_f / 1e9 / peak, 4),
            "getrf_hbm_gbps": round(byt / t_f / 1e6, 1), "getrf_hbm_frac": round(byt / t_f / 1e6 / PEAK_HBM, 4),
-           "tuned": {"nb": nb, "threads": nt}}
+           "tuned" if trial_ms > 0 else "config": {"nb": nb, "threads": nt}}
     plan.close()
     return out, ns, nrhs
 

@@ -311,7 +311,7 @@ template <> __device__ __forceinline__ float word_value<float>(int words, int l)
 // flight.  Measured, 64 columns of FP64 (before: the whole row exchanged and
 // updated in every column, agent-scope stores): 512 rows 214 -> 95 us, 128
 // rows 200 -> 69, 16384 rows on XCD 0 beside the update 276 -> 149; 32 columns
-// of 1024 rows 120 -> 64.
+// of 1024 rows 120 -> 59.
 template <class T, int W, int NTH, bool MULTI>
 struct LeafLds {
   static constexpr int NW = NTH / 64;
